@@ -7,9 +7,12 @@ build command, as operators.library does for the reference's DLLs (src/wan_dit_l
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parents[1] / "lib" / "libwdl.so"
+HOST_PATH = LIB_PATH.with_name("wdl_host.so")
 
 c_i64 = ctypes.c_int64
 c_int = ctypes.c_int
@@ -93,6 +96,24 @@ def library() -> ctypes.CDLL:
             fn.restype = RESTYPES.get(name, c_int)
         _LIB = lib
     return _LIB
+
+
+_HOST = None
+
+
+def host():
+    """The native launchers (host/launch.cpp) over the same library: lib/wdl_host.so, bound to LIB_PATH."""
+    global _HOST
+    if _HOST is None:
+        library()
+        if not HOST_PATH.exists():
+            raise FileNotFoundError(f"{HOST_PATH} is not built: python -m wdl.build (or __graft_entry__.build())")
+        loader = importlib.machinery.ExtensionFileLoader("wdl_host", str(HOST_PATH))
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("wdl_host", loader))
+        loader.exec_module(module)
+        module.bind(str(LIB_PATH))
+        _HOST = module
+    return _HOST
 
 
 def exported_symbols() -> list[str]:

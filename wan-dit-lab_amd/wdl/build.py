@@ -21,6 +21,8 @@ ROOT = Path(__file__).resolve().parents[1]  # wan-dit-lab_amd/
 CSRC = ROOT / "csrc"
 OBJ = ROOT / "_build"
 LIB = ROOT / "lib" / "libwdl.so"
+HOST_SRC = ROOT / "host" / "launch.cpp"
+HOST = ROOT / "lib" / "wdl_host.so"
 ARCH = "gfx950"
 
 FLAGS = [
@@ -74,5 +76,26 @@ def build(force: bool = False, jobs: int | None = None) -> Path:
     return LIB
 
 
+def build_host() -> Path:
+    """Compiles the native launchers (host/launch.cpp, against torch's headers) into lib/wdl_host.so."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    HOST.parent.mkdir(exist_ok=True)
+    tmp = HOST.with_suffix(".so.tmp")
+    includes = [str(ROOT.parent / "include"), *cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
+    cmd = ["g++", "-O2", "-std=c++17", "-shared", "-fPIC", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-DTORCH_EXTENSION_NAME=wdl_host", *(f for i in includes for f in ("-isystem", i)), str(HOST_SRC), "-o", str(tmp),
+           *(f"-L{p}" for p in cpp_extension.library_paths()), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
+    run = subprocess.run(cmd, capture_output=True, text=True)
+    if run.returncode != 0:
+        raise RuntimeError(f"g++ failed for {HOST_SRC.name}:\n{run.stdout}\n{run.stderr}")
+    os.replace(tmp, HOST)
+    return HOST
+
+
 if __name__ == "__main__":
     print(build(force="--force" in sys.argv))
+    print(build_host())

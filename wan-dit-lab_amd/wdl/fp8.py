@@ -12,7 +12,7 @@ from __future__ import annotations
 import torch
 
 from wdl import _lib
-from wdl.ops import ptr, stream_of, workspace
+from wdl.ops import stream_of, workspace
 
 FP8 = torch.float8_e4m3fn
 FP8_MAX = 448.0
@@ -35,17 +35,8 @@ def quantize_padded(x: torch.Tensor, rows: bool, pad: int = ROWS_PAD):
     (rows) or [1] (tensor)), Mp = ceil(M / pad) * pad."""
     if x.dim() != 2 or x.stride(1) != 1:
         raise ValueError("x must be a [M, K] matrix with contiguous rows")
-    M, K = x.shape
-    Mp = (M + pad - 1) // pad * pad
-    q = torch.empty(Mp, K, device=x.device, dtype=torch.uint8)
-    scale = torch.empty(Mp if rows else 1, device=x.device, dtype=torch.float32)
-    ws = None
-    if not rows:
-        n = _lib.library().wdl_fp8_quantize_workspace_floats(M, K)
-        ws = torch.empty(n, device=x.device, dtype=torch.float32)
-    _lib.call("wdl_fp8_quantize", ptr(x), _dtype_code(x), x.stride(0), M, K, Mp, int(rows), ptr(q), ptr(scale),
-              ptr(ws), stream_of(x))
-    return q, scale
+    _dtype_code(x)  # TypeError for other types
+    return _lib.host().fp8_quantize(x, bool(rows), pad, stream_of(x))
 
 
 def quantize(X: torch.Tensor):
@@ -75,12 +66,9 @@ def gemm(q: torch.Tensor, x_scale: torch.Tensor, M: int, w_codes: torch.Tensor, 
     if w_codes.shape[1] != K or N % 128 or K % 64:
         raise ValueError(f"fp8 GEMM needs [N, K] weights with N % 128 == 0 and K % 64 == 0, got {tuple(w_codes.shape)}")
     b = None if bias is None else bias.to(torch.bfloat16).contiguous()
-    out = torch.empty(M, N, device=q.device, dtype=torch.bfloat16)
     nbytes = _lib.library().wdl_fp8_gemm_workspace_bytes(Mp, N, K) if stream_k else 0
     ws = workspace(_FP8_GEMM_WS, q.device, nbytes) if nbytes else None
-    _lib.call("wdl_fp8_gemm", ptr(q), ptr(x_scale), ptr(w_codes.view(torch.uint8)), ptr(w_scale), ptr(b), M, Mp, N,
-              K, int(rows), ptr(out), out.stride(0), ptr(ws), stream_of(q))
-    return out
+    return _lib.host().fp8_gemm(q, x_scale, M, w_codes, w_scale, b, bool(rows), ws, stream_of(q))
 
 
 def weight_only_gemm(x: torch.Tensor, w_codes: torch.Tensor, w_scale: torch.Tensor, bias: torch.Tensor | None,
@@ -114,9 +102,7 @@ def weight_only_gemm(x: torch.Tensor, w_codes: torch.Tensor, w_scale: torch.Tens
         gate = gate.float().contiguous()
     elif out is None:
         out = torch.empty(M, N, device=x.device, dtype=torch.bfloat16)
-    _lib.call("wdl_fp8wo_gemm", ptr(x), x.stride(0), ptr(w_codes.view(torch.uint8)), ptr(w_scale),
-              int(w_scale.numel() == N and N > 1), ptr(b), M, N, K, ptr(out), out.stride(0), 0 if gate is None else 2,
-              ptr(gate), stream_of(x))
+    _lib.host().fp8wo_gemm(x, w_codes, w_scale, b, out, gate, stream_of(x))
     return out
 
 

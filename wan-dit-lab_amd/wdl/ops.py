@@ -15,11 +15,13 @@ import torch
 
 from wdl import _lib
 
-DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2, torch.float64: 3}
-
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current stream of t's GPU, as a handle."""
+    d = t.device
+    if d.type != "cuda":
+        raise ValueError(f"a tensor on the GPU is needed, got one on {d}")
+    return torch._C._cuda_getCurrentRawStream(d.index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
@@ -31,12 +33,9 @@ def ptr(t: torch.Tensor | None) -> int | None:
 @torch.library.custom_op("wdl::store_kv_fp8", mutates_args=("cache_k", "cache_ks", "cache_v", "cache_vs"))
 def store_kv_fp8_op(k: torch.Tensor, v: torch.Tensor, cache_k: torch.Tensor, cache_ks: torch.Tensor,
                     cache_v: torch.Tensor, cache_vs: torch.Tensor, at: int) -> None:
-    b, n, h, d = k.shape
     if k.numel() == 0:
         return
-    _lib.call("wdl_kv_append_fp8", ptr(k), DTYPE_CODE[k.dtype], _lib.i64s(k.stride()), ptr(v), DTYPE_CODE[v.dtype],
-              _lib.i64s(v.stride()), b, n, h, d, ptr(cache_k), ptr(cache_ks), ptr(cache_v), ptr(cache_vs),
-              cache_k.shape[1], at, stream_of(k))
+    _lib.host().kv_append(k, v, cache_k, cache_ks, cache_v, cache_vs, at, stream_of(k))
 
 
 @store_kv_fp8_op.register_fake
@@ -67,18 +66,12 @@ def act_quant_launch(x, smooth, proj_down_t, qshift=0.0, unsigned=False, *, ln=N
     or None).
     ln: dict(shift, scale, weight, bias, eps, partials) fuses LayerNorm + modulation; partials: the LayerNorm chunk
     partials of x (fp32 [M, K / 32, 2], as gemm_launch's ln_out writes them), or None to form them here."""
-    M, K = x.shape
-    Mp = padded_rows(M)
-    q = torch.empty(Mp // BLOCK, K // 64, BLOCK, ROW6, device=x.device, dtype=torch.uint8)
-    ascales = torch.empty(K // 64, Mp, device=x.device, dtype=torch.bfloat16)
-    lora = None if proj_down_t is None else torch.empty(Mp, RANK, device=x.device, dtype=torch.float32)
-    ln = ln or {}
-    ws = torch.empty(_lib.library().wdl_act_quant_workspace_floats(Mp, K), device=x.device, dtype=torch.float32)
-    _lib.call("wdl_act_quant_w4", ptr(x), x.stride(0), M, K, ptr(smooth), float(qshift), int(unsigned),
-              ptr(proj_down_t), RANK, ptr(q), ptr(ascales), ptr(lora), Mp, ptr(ln.get("shift")), ptr(ln.get("scale")),
-              ptr(ln.get("weight")), ptr(ln.get("bias")), int(bool(ln)), float(ln.get("eps", 1e-6)),
-              ptr(ln.get("partials")), ptr(v_out), ptr(ws), stream_of(x))
-    return q, ascales, lora
+    if not ln:
+        return _lib.host().act_quant(x, smooth, proj_down_t, qshift, unsigned, False, None, None, None, None, 1e-6, None,
+                                     v_out, stream_of(x))
+    return _lib.host().act_quant(x, smooth, proj_down_t, qshift, unsigned, True, ln.get("shift"), ln.get("scale"),
+                                 ln.get("weight"), ln.get("bias"), ln.get("eps", 1e-6), ln.get("partials"), v_out,
+                                 stream_of(x))
 
 
 # ---- the GEMM's operand format (tile-blocked fp6 codes): weights w in [-8, 7] as e3m2 codes of 2w, activations
@@ -243,8 +236,7 @@ def gemm_launch(q, ascales, lora, wcodes, wscales, proj_up, bias, M, out, epilog
     if ln_out is not None and (ln_out.dtype != torch.float32 or not ln_out.is_contiguous() or
                                ln_out.numel() < M * (N // 32) * 2 or out.shape[-1] != N):
         raise ValueError(f"ln_out: a contiguous fp32 [{M}, {N // 32}, 2] buffer for whole output rows of {N}")
-    _lib.call("wdl_w4a4_gemm", ptr(q), ptr(ascales), ptr(wcodes), ptr(wscales), ptr(lora), ptr(proj_up), ptr(bias),
-              M, Mp, N, K, RANK, ptr(out), out.stride(0), epilogue, ptr(gate), ptr(ln_out), ptr(ws), stream_of(q))
+    _lib.host().gemm(q, ascales, lora, wcodes, wscales, proj_up, bias, M, out, epilogue, gate, ln_out, ws, stream_of(q))
     return out
 
 
@@ -256,22 +248,13 @@ def gelu_quant_launch(q, ascales, lora, wcodes, wscales, proj_up, bias, M, smoot
     wscales = cached_scale_pairs(wscales)
     if q.dim() != 4 or wcodes.dim() != 4 or q.shape[2:] != (BLOCK, ROW6) or wcodes.shape[2:] != (BLOCK, ROW6):
         raise ValueError("the W4A4 GEMM takes tile-blocked fp6 operands [rows/128, K/64, 128, 48]")
-    Mp, K = q.shape[0] * BLOCK, q.shape[1] * 64
     N = wcodes.shape[0] * BLOCK
     if wcodes.shape[1] != q.shape[1]:
-        raise ValueError(f"weight codes {tuple(wcodes.shape)} do not match activations of width {K}")
+        raise ValueError(f"weight codes {tuple(wcodes.shape)} do not match activations of width {q.shape[1] * 64}")
     if smooth2.shape != (N,) or proj_down2_t.shape != (RANK, N):
         raise ValueError(f"smooth2 must be [{N}] and proj_down2 [{RANK}, {N}] for a hidden layer of {N}")
-    dev = q.device
-    q2 = torch.empty(Mp // BLOCK, N // 64, BLOCK, ROW6, device=dev, dtype=torch.uint8)
-    asc2 = torch.empty(N // 64, Mp, device=dev, dtype=torch.bfloat16)
-    lora2 = torch.empty(Mp, RANK, device=dev, dtype=torch.float32)
-    ws = torch.empty(_lib.library().wdl_w4a4_gemm_gelu_quant_workspace_floats(Mp, N), device=dev,
-                     dtype=torch.float32)
-    _lib.call("wdl_w4a4_gemm_gelu_quant", ptr(q), ptr(ascales), ptr(wcodes), ptr(wscales), ptr(lora), ptr(proj_up),
-              ptr(bias), M, Mp, N, K, RANK, ptr(smooth2), ptr(proj_down2_t), ptr(q2), ptr(asc2), ptr(lora2), ptr(ws),
-              stream_of(q))
-    return q2, asc2, lora2
+    return _lib.host().gelu_quant(q, ascales, lora, wcodes, wscales, proj_up, bias, M, smooth2, proj_down2_t,
+                                  stream_of(q))
 
 
 @torch.library.custom_op("wdl::act_quant_w4", mutates_args=())
@@ -353,16 +336,8 @@ def qk_norm_rope_launch(q, k, wq, wk, freq, grid, start_frame, eps=1e-6, q_out=N
     """q, k bf16 [M, H*128] (row-strided views allowed) -> RMSNorm(all heads) + 3D RoPE, bf16 [M, H*128] each.
     wq / wk None: that input is only rotated; k None: q alone (returns (q_out, None)). freq: contiguous fp32 or
     fp64 [2, positions, 64]."""
-    M, C = q.shape
     f, h, w = (int(v) for v in grid)
-    q_out = torch.empty(M, C, device=q.device, dtype=torch.bfloat16) if q_out is None else q_out
-    if k is not None and k_out is None:
-        k_out = torch.empty(M, C, device=q.device, dtype=torch.bfloat16)
-    code = {torch.float32: 0, torch.float64: 3}[freq.dtype]
-    _lib.call("wdl_qk_norm_rope", ptr(q), q.stride(0), ptr(k), 0 if k is None else k.stride(0), ptr(wq), ptr(wk),
-              ptr(freq), code, freq.shape[1], M, C // 128, f, h, w, int(start_frame), float(eps), ptr(q_out),
-              ptr(k_out), q_out.stride(0), stream_of(q))
-    return q_out, k_out
+    return _lib.host().qk_norm_rope(q, k, wq, wk, freq, f, h, w, int(start_frame), eps, q_out, k_out, stream_of(q))
 
 
 def quant_q_launch(x, heads):
@@ -409,6 +384,20 @@ def sage_prep_launch(cache_k, cache_ks, cache_v, cache_vs, k, v, at, want_stats=
     (wdl_sage_prep_cached_append: the bytes and scales of wdl_kv_append_fp8)."""
     n = k.shape[0]
     H = k.shape[1] // 128
+    if cache_stats is not None:
+        if heads is not None or tokens is not None:
+            raise ValueError("cache statistics are for the unmapped cache")
+        if cache_stats.shape != (2, H, 128) or cache_stats.dtype != torch.float32 or not cache_stats.is_contiguous():
+            raise ValueError(f"cache statistics must be contiguous fp32 [2, {H}, 128]")
+    elif append:
+        raise ValueError("append runs with the cache statistics")
+    if heads is None and tokens is None:
+        k_i8, k_sc, v_f8, v_sc, k_mean = _lib.host().sage_prep(cache_k, cache_ks, cache_v, cache_vs, k, v, at, SPLITS,
+                                                               cache_stats, append, stream_of(k))
+        out = dict(k=k_i8, k_scale=k_sc, v=v_f8, v_scale=v_sc)
+        if want_stats:
+            out["k_mean"] = k_mean
+        return out
     Hc = cache_k.shape[2]
     L = at + n
     Lp = (L + 63) // 64 * 64
@@ -419,25 +408,9 @@ def sage_prep_launch(cache_k, cache_ks, cache_v, cache_vs, k, v, at, want_stats=
     v_f8 = torch.empty(H, 128, Lp, device=dev, dtype=torch.uint8)
     k_mean = torch.empty(H, 128, device=dev, dtype=torch.float32)
     v_sc = torch.empty(H, 128, device=dev, dtype=torch.float32)
-    if cache_stats is not None:
-        if heads is not None or tokens is not None:
-            raise ValueError("cache statistics are for the unmapped cache")
-        if cache_stats.shape != (2, H, 128) or cache_stats.dtype != torch.float32 or not cache_stats.is_contiguous():
-            raise ValueError(f"cache statistics must be contiguous fp32 [2, {H}, 128]")
-        _lib.call("wdl_sage_prep_cached_append" if append else "wdl_sage_prep_cached", ptr(cache_k), ptr(cache_ks),
-                  ptr(cache_v), ptr(cache_vs), cache_k.shape[1], ptr(k), k.stride(0), ptr(v), v.stride(0), H, at, n,
-                  ptr(cache_stats), SPLITS, ptr(ws), ptr(k_i8), ptr(k_sc), ptr(v_f8), ptr(k_mean), ptr(v_sc),
-                  stream_of(k))
-    elif append:
-        raise ValueError("append runs with the cache statistics")
-    elif heads is None and tokens is None:
-        _lib.call("wdl_sage_prep", ptr(cache_k), ptr(cache_ks), ptr(cache_v), ptr(cache_vs), cache_k.shape[1],
-                  ptr(k), k.stride(0), ptr(v), v.stride(0), H, at, n, SPLITS, ptr(ws), ptr(k_i8), ptr(k_sc),
-                  ptr(v_f8), ptr(k_mean), ptr(v_sc), stream_of(k))
-    else:
-        _lib.call("wdl_sage_prep_mapped", ptr(cache_k), ptr(cache_ks), ptr(cache_v), ptr(cache_vs),
-                  cache_k.shape[1], Hc, ptr(heads), ptr(tokens), ptr(k), k.stride(0), ptr(v), v.stride(0), H, at, n,
-                  SPLITS, ptr(ws), ptr(k_i8), ptr(k_sc), ptr(v_f8), ptr(k_mean), ptr(v_sc), stream_of(k))
+    _lib.call("wdl_sage_prep_mapped", ptr(cache_k), ptr(cache_ks), ptr(cache_v), ptr(cache_vs), cache_k.shape[1], Hc,
+              ptr(heads), ptr(tokens), ptr(k), k.stride(0), ptr(v), v.stride(0), H, at, n, SPLITS, ptr(ws), ptr(k_i8),
+              ptr(k_sc), ptr(v_f8), ptr(k_mean), ptr(v_sc), stream_of(k))
     out = dict(k=k_i8, k_scale=k_sc, v=v_f8, v_scale=v_sc)
     if want_stats:
         out["k_mean"] = k_mean
@@ -504,19 +477,14 @@ def sage_attn_q16_launch(Q, prep, L, sm_scale, out=None, frame_tokens=0):
     H = Q.shape[1] // 128
     if Q.dtype != torch.bfloat16 or Q.dim() != 2 or Q.shape[1] % 128 or Q.stride(1) != 1:
         raise ValueError("sage_attn_q16: Q must be bf16 [n, H*128] with unit column stride")
-    if out is None:
-        out = torch.empty(n, H * 128, device=Q.device, dtype=torch.bfloat16)
+    ws = None
     if frame_tokens:
         if not isinstance(frame_tokens, int) or frame_tokens < 0 or n > L:
             raise ValueError("sage_attn_q16: frame_tokens must be a positive int and the queries among the keys")
-        _lib.call("wdl_sage_attn_q16_framed", ptr(Q), Q.stride(0), ptr(prep["k"]), ptr(prep["k_scale"]),
-                  ptr(prep["v"]), ptr(prep["v_scale"]), n, L, H, float(sm_scale), frame_tokens, ptr(out),
-                  out.stride(0), 0, stream_of(Q))
-        return out
-    ws = workspace(_ATTN_WS, Q.device, _lib.library().wdl_sage_attn_workspace_bytes(n, L, H))
-    _lib.call("wdl_sage_attn_q16", ptr(Q), Q.stride(0), ptr(prep["k"]), ptr(prep["k_scale"]), ptr(prep["v"]),
-              ptr(prep["v_scale"]), n, L, H, float(sm_scale), ptr(out), out.stride(0), ptr(ws), stream_of(Q))
-    return out
+    else:
+        ws = workspace(_ATTN_WS, Q.device, _lib.library().wdl_sage_attn_workspace_bytes(n, L, H))
+    return _lib.host().sage_attn_q16(Q, prep["k"], prep["k_scale"], prep["v"], prep["v_scale"], L, sm_scale, out,
+                                     int(frame_tokens), ws, stream_of(Q))
 
 
 def attn_bf16_prep_launch(K, V):
@@ -534,18 +502,11 @@ def attn_bf16_prep_launch(K, V):
     return dict(kp=kp, vp=vp, L=L, heads=H)
 
 
-def _attn_bf16_into(Q, kp, vp, L, H, sm_scale, out):
-    _lib.call("wdl_attn_bf16", ptr(Q), Q.stride(0), ptr(kp), ptr(vp), Q.shape[0], L, H, float(sm_scale), ptr(out),
-              out.stride(0), stream_of(Q))
-    return out
-
-
 @torch.library.custom_op("wdl::attn_bf16", mutates_args=())
 def attn_bf16(q: torch.Tensor, kp: torch.Tensor, vp: torch.Tensor, keys: int, sm_scale: float) -> torch.Tensor:
     """softmax(q K^T sm_scale) V in bf16 with an fp32 softmax (the reference's SDPA on bf16 operands) for q bf16
     [n, H*128] over the `keys` keys laid out by attn_bf16_prep_launch (kp, vp) -> bf16 [n, H*128]."""
-    out = torch.empty(q.shape, device=q.device, dtype=torch.bfloat16)
-    return _attn_bf16_into(q, kp, vp, keys, q.shape[1] // 128, sm_scale, out)
+    return _lib.host().attn_bf16(q, kp, vp, keys, sm_scale, None, stream_of(q))
 
 
 @attn_bf16.register_fake
@@ -562,7 +523,7 @@ def attn_bf16_launch(Q, prep, sm_scale, out=None):
         raise ValueError(f"attn_bf16: Q must be bf16 [n, {H * 128}] with unit column stride")
     if out is None:
         return attn_bf16(Q, prep["kp"], prep["vp"], prep["L"], float(sm_scale))
-    return _attn_bf16_into(Q, prep["kp"], prep["vp"], prep["L"], H, sm_scale, out)
+    return _lib.host().attn_bf16(Q, prep["kp"], prep["vp"], prep["L"], sm_scale, out, stream_of(Q))
 
 
 @torch.library.custom_op("wdl::sage_kv_attend", mutates_args=())

@@ -13,7 +13,7 @@ from __future__ import annotations
 import torch
 
 from wdl import _lib
-from wdl.ops import DTYPE_CODE, qk_norm_rope_launch, stream_of
+from wdl.ops import qk_norm_rope_launch, stream_of
 
 
 def rope(pos_count: int, pos_dim: int) -> torch.Tensor:
@@ -63,14 +63,7 @@ def rope3d_rotate(x: torch.Tensor, freq: torch.Tensor, grid_key: str, start: int
     """wan_dit_lab::rope3d_rotate (kernels/rope_triton.py:66-81) on wdl_rope3d_rotate: x [B, L, H, dim] (any strides)
     turned by the 3D RoPE angles of the grids in grid_key ("f,h,w,f,h,w,..."), by -angle when inverse; a new
     contiguous tensor of output_dtype."""
-    out = torch.empty(x.shape, device=x.device, dtype=output_dtype)
-    if x.numel():
-        grids = [int(v) for v in grid_key.split(",")]
-        B, L, H, dim = x.shape
-        _lib.call("wdl_rope3d_rotate", x.data_ptr(), DTYPE_CODE[x.dtype], _lib.i64s(x.stride()), freq.data_ptr(),
-                  DTYPE_CODE[freq.dtype], _lib.i64s(freq.stride()), freq.shape[1], B, L, H, dim, _lib.i32s(grids),
-                  int(start), int(bool(inverse)), out.data_ptr(), DTYPE_CODE[output_dtype], stream_of(x))
-    return out
+    return _lib.host().rope3d(x, freq, [int(v) for v in grid_key.split(",")], start, inverse, output_dtype, stream_of(x))
 
 
 @rope3d_rotate.register_fake

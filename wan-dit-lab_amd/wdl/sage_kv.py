@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import torch
 
+from wdl import _lib
 from wdl.ops import (quant_q_launch, sage_attn_launch, sage_kv_append_attend_cached, sage_kv_attend,
                      sage_kv_attend_cached, sage_prep_launch)
 
@@ -63,13 +64,15 @@ def attend(Q, cache_k, cache_ks, cache_v, cache_vs, at, K, V, sm_scale=None, hea
     tokens beside them. append (with cache_stats, not with frame_tokens): K, V also go into cache rows at .. at + n
     (KVCache.store's store_kv_fp8, causal.py:177-181) inside the preparation pass; its requirements are checked
     first, and a broken one raises before anything is written."""
-    _check(Q, cache_k, cache_ks, cache_v, cache_vs, at, K, V, heads, tokens)
+    if heads is not None or tokens is not None or type(at) is not int or torch.compiler.is_compiling() or \
+            not _lib.host().attend_valid(Q, cache_k, cache_ks, cache_v, cache_vs, at, K, V):
+        _check(Q, cache_k, cache_ks, cache_v, cache_vs, at, K, V, heads, tokens)
     if append:
-        from wdl.cache_fp8 import _refusal
+        from wdl.cache_fp8 import refusal
 
         if cache_stats is None or frame_tokens:
             raise ValueError("append runs with the cache statistics and without frame_tokens")
-        refused = _refusal(K, V, cache_k, cache_ks, cache_v, cache_vs, at)
+        refused = refusal(K, V, cache_k, cache_ks, cache_v, cache_vs, at)
         if refused is not None:
             kind, message = refused
             raise kind(message)
