@@ -74,3 +74,28 @@ def test_weight_only_residual_epilogue_and_module(gpu):
     assert torch.equal(mod.weight.cpu().view(torch.uint8), wq.view(torch.uint8))
     got = mod(x.cuda()[None]).cpu()[0]
     assert check(got, x, wq, ws, b, y) >= 0.995
+
+
+@pytest.mark.parametrize("M,N,K", [(2047, 2048, 64), (2049, 2304, 192), (127, 32768, 64), (128, 32512, 64),
+                                   (129, 16640, 128)])
+def test_weight_only_tiles_at_their_edges(gpu, M, N, K):
+    """Both tile sizes around the line between them (128 tiles of 256 x 128 on 256 CUs), one token short of and past a
+    tile, one to three stages of K, all 254 finite codes among the weights, and the gated residual into a strided
+    output: the bars of the tests above."""
+    from wdl import fp8
+
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).to(BF)
+    codes = torch.arange(256, dtype=torch.uint8)
+    codes = codes[(codes & 127) != 127].repeat(N * K // 254 + 1)[:N * K]
+    wq = codes[torch.randperm(N * K, generator=g)].reshape(N, K).view(torch.float8_e4m3fn)
+    ws, b = torch.rand(N, 1, generator=g) * 0.01 + 0.001, torch.randn(N, generator=g).to(BF)
+    want = ofp8.w8a16_linear(x, wq, ws, b)
+    args = (x.cuda(), wq.cuda(), ws.reshape(-1).cuda(), b.cuda())
+    got = fp8.weight_only_gemm(*args)
+    assert check(got.cpu(), x, wq, ws, b, want) >= 0.995
+    res, gate = torch.randn(M, N + 4, generator=g).to(BF), torch.rand(N, generator=g)
+    out = res.cuda()
+    fp8.weight_only_gemm(*args, out=out[:, :N], gate=gate.cuda())
+    assert torch.equal(out.cpu()[:, :N], (res[:, :N].float() + got.cpu().float() * gate).to(BF))
+    assert torch.equal(out.cpu()[:, N:], res[:, N:])
