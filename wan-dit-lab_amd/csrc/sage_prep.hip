@@ -1,15 +1,14 @@
 // Sage-2 preparation read straight from the FP8 KV cache and the chunk's own bf16 K/V (kernels/sage_kv.py:28-173).
 //
 // Token t of a call: t < at comes from the cache (e4m3 value * its fp32 row scale), at <= t < L = at + n from the
-// chunk (bf16), t >= L is zero. Three launches:
+// chunk (bf16), t >= L is zero. Two launches:
 //   colstats   (grid H x S): per split s of the tokens, partial sums of K and maxima of |V| per (head, channel),
 //              each in a fixed order (16 token lanes, then the lanes in order);
-//   finalize   (grid H):     k_mean = (sum over splits, in order) / L;  v_scale = max(max |V|, 1e-8) / 2.25;
-//              with cached statistics of tokens [0, at) (wdl_sage_cache_stats: their sums and maxima, formed the
-//              same way over splits of [0, at)) the splits cover only the chunk's tokens and the sum starts from
-//              the cached one;
-//   quant_kv   (grid blocks x H): K - mean to int8 with one scale per group g = 0..3 of each 64-token block (tokens
-//              8i + 2g, 8i + 2g + 1): scale = max|x| / 127 + 1e-7, q = trunc(x / scale +- 0.5);
+//   quant_kv   (grid blocks x H): first, per workgroup, k_mean = (sum over splits, in order) / L and v_scale = max(max
+//              |V|, 1e-8) / 2.25 of its head; with cached statistics of tokens [0, at) (wdl_sage_cache_stats: their sums
+//              and maxima, formed the same way over splits of [0, at)) the splits cover only the chunk's tokens and the
+//              sum starts from the cached one. Then K - mean to int8 with one scale per group g = 0..3 of each 64-token
+//              block (tokens 8i + 2g, 8i + 2g + 1): scale = max|x| / 127 + 1e-7, q = trunc(x / scale +- 0.5);
 //              V / v_scale to e4m3, stored per (head, channel) along the tokens in wdl's order: within a
 //              64-token block, position 32 * ((t % 8) / 4) + 4 * (t / 8) + t % 4 holds token t (the key order one
 //              lane half of the transposed QK^T MFMA tile produces, so P feeds the PV MFMA unshuffled).
@@ -135,38 +134,49 @@ __global__ __launch_bounds__(256) void colstats_kernel(Src k, Src v, int64_t H, 
     }
 }
 
-// base: null, or cached statistics [2][H][D] (K sums, |V| maxima) the splits' values are added to; raw: write the
-// sums and maxima into k_mean (as [2][H][D]) instead of the mean and v_scale
-__global__ void finalize_kernel(const float* part_k, const float* part_v, int S, int64_t H, int64_t L, float* k_mean,
-                                float* v_scale, const float* base, int raw) {
-    const int64_t h = blockIdx.x;
-    const int d = threadIdx.x;
-    // the splits in increasing order; the loads of a batch of 16 are all issued before the first add (one memory
-    // round trip per batch, not one per split)
+// The splits' partial sums (or maxima) of one column added in increasing order onto `from`; the loads of a batch of 16
+// are all issued before the first is used (one memory round trip per batch, not one per split).
+template <typename Op>
+__device__ __forceinline__ float over_splits(const float* part, int S, int64_t stride, float from, Op op) {
     constexpr int BATCH = 16;
-    float a = base ? base[h * D + d] : 0.0f, m = base ? base[(H + h) * D + d] : 0.0f;
     for (int s0 = 0; s0 < S; s0 += BATCH) {
-        float pk[BATCH], pv[BATCH];
+        float p[BATCH];
 #pragma unroll
-        for (int j = 0; j < BATCH; ++j) {
-            const bool in = s0 + j < S;
-            pk[j] = in ? part_k[((s0 + j) * H + h) * D + d] : 0.0f;
-            pv[j] = in ? part_v[((s0 + j) * H + h) * D + d] : 0.0f;
-        }
+        for (int j = 0; j < BATCH; ++j) p[j] = s0 + j < S ? part[(s0 + j) * stride] : 0.0f;
 #pragma unroll
         for (int j = 0; j < BATCH; ++j)
-            if (s0 + j < S) {
-                a = a + pk[j];
-                m = fmaxf(m, pv[j]);
-            }
+            if (s0 + j < S) from = op(from, p[j]);
     }
-    if (raw) {
-        k_mean[h * D + d] = a;
-        k_mean[(H + h) * D + d] = m;
-        return;
+    return from;
+}
+struct Add {
+    __device__ float operator()(float a, float b) const { return a + b; }
+};
+struct Max {
+    __device__ float operator()(float a, float b) const { return fmaxf(a, b); }
+};
+
+// The column statistics of a call: the splits' partials, and null or the cached statistics [2][H][D] (K sums, |V| maxima)
+// that they are added to.
+struct Stats {
+    const float* part_k;
+    const float* part_v;
+    const float* base;
+    int S;
+    // K sum / |V| maximum of column i = h D + d
+    __device__ __forceinline__ float sum(int64_t i, int64_t HD) const {
+        return over_splits(part_k + i, S, HD, base ? base[i] : 0.0f, Add{});
     }
-    k_mean[h * D + d] = a / float(L);
-    v_scale[h * D + d] = fmaxf(m, 1e-8f) / 2.25f;
+    __device__ __forceinline__ float max(int64_t i, int64_t HD) const {
+        return over_splits(part_v + i, S, HD, base ? base[HD + i] : 0.0f, Max{});
+    }
+};
+
+// wdl_sage_cache_stats: the sums and maxima themselves, [2][H][D]
+__global__ void finalize_kernel(Stats st, int64_t HD, float* out) {
+    const int64_t i = int64_t(blockIdx.x) * D + threadIdx.x;
+    out[i] = st.sum(i, HD);
+    out[HD + i] = st.max(i, HD);
 }
 
 __device__ __forceinline__ int v_position(int t) { return 32 * ((t % 8) / 4) + 4 * (t / 8) + t % 4; }
@@ -241,7 +251,7 @@ struct Append {
 };
 
 __global__ __launch_bounds__(256) void quant_kv_kernel(Src k, Src v, int64_t H, int64_t at, int64_t L, int64_t Lpad,
-                                                       const float* k_mean, const float* v_scale, int8_t* k_out,
+                                                       Stats st, float* k_mean, float* v_scale, int8_t* k_out,
                                                        float* k_scale, uint8_t* v_out, Append app) {
     __shared__ float gmax[64][4];
     __shared__ __attribute__((aligned(16))) uint8_t vt[D][64 + 4];  // codes [channel][position], 4-byte rows
@@ -249,11 +259,20 @@ __global__ __launch_bounds__(256) void quant_kv_kernel(Src k, Src v, int64_t H, 
     const int64_t blk = blockIdx.x, h = blockIdx.y;
     const int t = threadIdx.x, tt = t / 4, dq = (t % 4) * 32;
     const int64_t tok = blk * 64 + tt;
-    if (t < D) {
-        stat[0][t] = k_mean[h * D + t];
-        const float vs = v_scale[h * D + t];
-        stat[1][t] = vs;
-        stat[2][t] = 1.0f / vs;
+    // the head's statistics from the splits' partials (16 KB from L2 per workgroup, beside its tokens' loads; a launch
+    // of its own for them took 4 - 5 us in front of this one); the first block keeps them for the caller
+    {
+        const int64_t i = h * D + t % D;
+        if (t < D) {
+            const float mean = st.sum(i, H * D) / float(L);
+            stat[0][t] = mean;
+            if (blk == 0) k_mean[i] = mean;
+        } else {
+            const float vs = fmaxf(st.max(i, H * D), 1e-8f) / 2.25f;
+            stat[1][t - D] = vs;
+            stat[2][t - D] = 1.0f / vs;
+            if (blk == 0) v_scale[i] = vs;
+        }
     }
     // all loads of this thread's token first (the block's source is uniform unless it straddles at or L)
     float fk[4][8], fv[4][8];
@@ -446,14 +465,10 @@ static int sage_prep_launch(const void* cache_k, const float* cache_ks, const vo
     const int64_t t0 = cache_stats ? at : 0;
     colstats_kernel<<<dim3(unsigned(heads), unsigned(splits)), 256, 0, stream>>>(sk, sv, heads, at, t0, L, splits,
                                                                                  part_k, part_v);
-    int rc = check_launch("sage_prep colstats");
-    if (rc) return rc;
-    finalize_kernel<<<unsigned(heads), D, 0, stream>>>(part_k, part_v, splits, heads, L, k_mean, v_scale, cache_stats,
-                                                       0);
-    rc = check_launch("sage_prep finalize");
+    const int rc = check_launch("sage_prep colstats");
     if (rc) return rc;
     quant_kv_kernel<<<dim3(unsigned(Lpad / 64), unsigned(heads)), 256, 0, stream>>>(
-        sk, sv, heads, at, L, Lpad, k_mean, v_scale, static_cast<int8_t*>(k_int8), k_scale,
+        sk, sv, heads, at, L, Lpad, Stats{part_k, part_v, cache_stats, splits}, k_mean, v_scale, static_cast<int8_t*>(k_int8), k_scale,
         static_cast<uint8_t*>(v_fp8), app);
     return check_launch("sage_prep quant_kv");
 }
@@ -495,7 +510,7 @@ extern "C" int wdl_sage_cache_stats(const void* cache_k, const float* cache_ks, 
                                                                                  part_k, part_v);
     const int rc = check_launch("sage_cache_stats colstats");
     if (rc) return rc;
-    finalize_kernel<<<unsigned(heads), D, 0, stream>>>(part_k, part_v, splits, heads, at, stats, nullptr, nullptr, 1);
+    finalize_kernel<<<unsigned(heads), D, 0, stream>>>(Stats{part_k, part_v, nullptr, splits}, heads * D, stats);
     return check_launch("sage_cache_stats finalize");
 }
 
