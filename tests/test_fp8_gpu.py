@@ -148,3 +148,43 @@ def test_shapes_outside_the_tiles_are_rejected(gpu):
     lin = torch.nn.Linear(256, 100, device="cuda", dtype=BF)
     with pytest.raises(ValueError):
         fp8.DynamicFp8Linear(lin)(torch.randn(3, 256, device="cuda", dtype=BF))
+
+
+@pytest.mark.parametrize("rows", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("what", ["plain", "huge", "tiny", "spread", "infinite", "nan"])
+def test_quantizers_codes_over_the_types_range(gpu, what, dtype, rows):
+    """Codes and scales against the oracle over the whole range of the type (quotients formed through the scale's
+    reciprocal), with infinities (finite values of that scale to 0) and NaN, for contiguous and strided rows, with
+    padding rows; 130 x 272 leaves a ragged last round of chunks."""
+    from oracle import fp8 as ofp8
+    from wdl import fp8
+
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(130, 272, generator=g)
+    if what in ("huge", "tiny"):
+        x *= 2.0 ** (120 if what == "huge" else -120)
+    if what == "spread":
+        x = torch.exp2(torch.randint(-149, 121, x.shape, generator=g).float()) * x.sign()
+        x[5], x[6] = 0.0, -0.0
+    if what == "infinite":
+        x[3, 5], x[7, 0] = float("inf"), -float("inf")
+    if what == "nan":
+        x[3, 5] = float("nan")
+    x = x.to(dtype)
+    if what == "nan":  # torch's maximum is NaN then; the kernel's is the largest number's
+        y = x.clone()
+        y[3, 5] = 0
+        want, scale = (ofp8.quantize_rows if rows else ofp8.quantize)(y)
+        want = want.view(torch.uint8)
+    else:
+        want, scale = (ofp8.quantize_rows if rows else ofp8.quantize)(x)
+        want = want.view(torch.uint8)
+    wide = torch.cat([x, x], 1).cuda()
+    for t in (x.cuda(), wide[:, :272]):
+        q, s = fp8.quantize_padded(t, rows=rows)
+        if what == "nan":  # a NaN of either sign
+            assert int(q[3, 5]) & 127 == 127
+            q[3, 5] = want[3, 5].item()
+        assert torch.equal(q[:130].cpu(), want) and not q[130:].any()
+        assert torch.equal(s[:130].cpu(), scale.reshape(-1)) if rows else float(s) == float(scale)

@@ -52,6 +52,12 @@ __device__ __forceinline__ void ld8<uint16_t>(const uint16_t* p, float* f) {
     for (int e = 0; e < 4; ++e) f[2 * e] = __uint_as_float(w[e] << 16), f[2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u);
 }
 
+// x / s for the quantizers' scale s (its reciprocal rs beside it): div_rn, the IEEE quotient wherever it does not round
+// to a zero code; an infinite s (an infinite |x|) takes the division itself (finite values: 0, infinite: NaN)
+__device__ __forceinline__ float quotient(float x, float s, float rs) {
+    return s < INFINITY ? div_rn(x, s, rs) : x / s;
+}
+
 // One workgroup of WPR waves per row, 8 values per lane and step, two steps in flight: the row's maximum (lanes,
 // then waves through LDS), then the codes from a second read of the row (from cache). The maximum is
 // order-independent, so the result is the same for any WPR.
@@ -95,11 +101,12 @@ __global__ __launch_bounds__(64 * WPR) void rows_kernel(const T* x, int64_t ldx,
     }
     const float s = fmaxf(amax, 1e-12f) / FP8_MAX;
     if (t == 0) scale[row] = s;
+    const float rs = 1.0f / s;
     auto codes = [&](int64_t cc) {
         float f[8];
         ld8<T>(xr + 8 * cc, f);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) f[e] = f[e] / s;
+        for (int e = 0; e < 8; ++e) f[e] = quotient(f[e], s, rs);
         qr[cc] = make_uint2(e4m3x4(f), e4m3x4(f + 4));
     };
     c = t;
@@ -110,25 +117,30 @@ __global__ __launch_bounds__(64 * WPR) void rows_kernel(const T* x, int64_t ldx,
     if (c < chunks) codes(c);
 }
 
-template <typename T>
+// Chunk i (8 values) of a [rows, K] matrix with row stride ldx. FLAT: ldx = K, so the chunks are consecutive (a 64-bit
+// division per chunk cost more than its eight quotients).
+template <bool FLAT, typename T>
+__device__ __forceinline__ const T* chunk_at(const T* x, int64_t ldx, int64_t k8, int64_t i) {
+    return FLAT ? x + 8 * i : x + (i / k8) * ldx + 8 * (i % k8);
+}
+
+constexpr int INFLIGHT = 4;  // chunks a thread has in flight
+
+template <typename T, bool FLAT>
 __global__ __launch_bounds__(256) void tensor_max_kernel(const T* x, int64_t ldx, int64_t M, int64_t K,
                                                          float* partial) {
     __shared__ float red[4];
     const int64_t k8 = K / 8, n8 = M * k8, stride = int64_t(gridDim.x) * 256;
     float amax = 0.0f;
-    int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    for (; i + stride < n8; i += 2 * stride) {  // two 16-byte loads of bf16 in flight
-        float f[8], g[8];
-        ld8<T>(x + (i / k8) * ldx + 8 * (i % k8), f);
-        ld8<T>(x + ((i + stride) / k8) * ldx + 8 * ((i + stride) % k8), g);
+    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n8; i += INFLIGHT * stride) {
+        float f[INFLIGHT][8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fmaxf(fabsf(f[e]), fabsf(g[e])));
-    }
-    if (i < n8) {
-        float f[8];
-        ld8<T>(x + (i / k8) * ldx + 8 * (i % k8), f);
+        for (int u = 0; u < INFLIGHT; ++u)  // past the end: the thread's first chunk again
+            ld8<T>(chunk_at<FLAT>(x, ldx, k8, i + u * stride < n8 ? i + u * stride : i), f[u]);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(f[e]));
+        for (int u = 0; u < INFLIGHT; ++u)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(f[u][e]));
     }
     amax = group_max<64>(amax);
     if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = amax;
@@ -136,7 +148,7 @@ __global__ __launch_bounds__(256) void tensor_max_kernel(const T* x, int64_t ldx
     if (threadIdx.x == 0) partial[blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
-template <typename T>
+template <typename T, bool FLAT>
 __global__ __launch_bounds__(256) void tensor_quant_kernel(const T* x, int64_t ldx, int64_t M, int64_t Mp, int64_t K,
                                                            const float* partial, int nparts, uint8_t* q, float* scale) {
     __shared__ float red[4];
@@ -147,28 +159,26 @@ __global__ __launch_bounds__(256) void tensor_quant_kernel(const T* x, int64_t l
     __syncthreads();
     const float s = fmaxf(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])), 1e-12f) / FP8_MAX;
     if (blockIdx.x == 0 && threadIdx.x == 0) scale[0] = s;
-    const int64_t k8 = K / 8, n8 = Mp * k8, stride = int64_t(gridDim.x) * 256;
-    auto codes = [&](int64_t i) {
-        const int64_t m = i / k8, c = i % k8;
-        uint2 w = make_uint2(0u, 0u);
-        if (m < M) {
-            float f[8];
-            ld8<T>(x + m * ldx + 8 * c, f);
+    const float rs = 1.0f / s;
+    const int64_t k8 = K / 8, n8 = M * k8, np8 = Mp * k8, stride = int64_t(gridDim.x) * 256;
+    uint2* const out = reinterpret_cast<uint2*>(q);  // [Mp, K] bytes, no gaps: chunk i is out[i]
+    int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    for (; i < n8; i += INFLIGHT * stride) {
+        float f[INFLIGHT][8];
+#pragma unroll
+        for (int u = 0; u < INFLIGHT; ++u)
+            ld8<T>(chunk_at<FLAT>(x, ldx, k8, i + u * stride < n8 ? i + u * stride : i), f[u]);
+#pragma unroll
+        for (int u = 0; u < INFLIGHT; ++u) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                f[e] = f[e] / s;
-                if constexpr (sizeof(T) == 2) f[e] = bf16_to_f32(f32_to_bf16(f[e]));
+                f[u][e] = quotient(f[u][e], s, rs);
+                if constexpr (sizeof(T) == 2) f[u][e] = bf16_to_f32(f32_to_bf16(f[u][e]));
             }
-            w = make_uint2(e4m3x4(f), e4m3x4(f + 4));
+            if (i + u * stride < n8) out[i + u * stride] = make_uint2(e4m3x4(f[u]), e4m3x4(f[u] + 4));
         }
-        reinterpret_cast<uint2*>(q + m * K)[c] = w;
-    };
-    int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    for (; i + stride < n8; i += 2 * stride) {
-        codes(i);
-        codes(i + stride);
     }
-    if (i < n8) codes(i);
+    for (i = n8 + int64_t(blockIdx.x) * 256 + threadIdx.x; i < np8; i += stride) out[i] = make_uint2(0u, 0u);
 }
 
 int tensor_blocks(int64_t M, int64_t K) {
@@ -188,12 +198,15 @@ int quantize(const void* xv, int64_t ldx, int64_t M, int64_t K, int64_t Mp, int 
         return check_launch("fp8_quantize rows");
     }
     const int nb = tensor_blocks(M, K);
+    const bool flat = ldx == K || M <= 1;
     if (M > 0) {
-        tensor_max_kernel<T><<<unsigned(nb), 256, 0, stream>>>(x, ldx, M, K, workspace);
+        if (flat) tensor_max_kernel<T, true><<<unsigned(nb), 256, 0, stream>>>(x, ldx, M, K, workspace);
+        else tensor_max_kernel<T, false><<<unsigned(nb), 256, 0, stream>>>(x, ldx, M, K, workspace);
         const int rc = check_launch("fp8_quantize tensor max");
         if (rc) return rc;
     }
-    tensor_quant_kernel<T><<<unsigned(nb), 256, 0, stream>>>(x, ldx, M, Mp, K, workspace, M > 0 ? nb : 0, qb, scale);
+    if (flat) tensor_quant_kernel<T, true><<<unsigned(nb), 256, 0, stream>>>(x, ldx, M, Mp, K, workspace, M > 0 ? nb : 0, qb, scale);
+    else tensor_quant_kernel<T, false><<<unsigned(nb), 256, 0, stream>>>(x, ldx, M, Mp, K, workspace, M > 0 ? nb : 0, qb, scale);
     return check_launch("fp8_quantize tensor");
 }
 
