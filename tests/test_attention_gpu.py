@@ -317,6 +317,30 @@ def test_qk_norm_rope_bit_exact(gpu, grid, start, M):
         assert torch.equal(got.cpu().reshape(1, M, H, 128), want)
 
 
+@pytest.mark.parametrize("table", ["fp32", "fp64"])
+@pytest.mark.parametrize("heads,grid,start,M,offset", [
+    (1, (1, 1, 1), 1023, 1, 0), (3, (2, 1, 7), 3, 15, 0), (5, (1, 5, 1), 0, 7, 1), (32, (2, 3, 5), 7, 33, 1),
+    (9, (0, 900, 1000), 0, 3, 0)])
+def test_qk_norm_rope_place_and_table_edges(gpu, table, heads, grid, start, M, offset):
+    """Odd head counts (a lane's chunks end early), one-line and one-column grids, padding rows, an odd row count, a table
+    that is not 16-byte aligned, and a grid of no frames whose lines and columns exceed the rows: bit-exact, fp32 and fp64."""
+    from wdl import rope
+
+    C = heads * 128
+    g = torch.Generator().manual_seed(M)
+    q, k = ((torch.randn(M, C, generator=g) * 2).to(torch.bfloat16) for _ in range(2))
+    w = (torch.rand(C, generator=g) + 0.5).to(torch.bfloat16)
+    freq = orope.freqs(128, 1024, torch.float64)
+    freq = freq.float() if table == "fp32" else freq
+    d = torch.empty(freq.numel() + offset, dtype=freq.dtype, device="cuda")[offset:].view(freq.shape)
+    d.copy_(freq)
+    Qo, Ko = rope.norm_rope(q.cuda(), k.cuda(), w.cuda(), w.cuda(), d, grid, start)
+    for x, got in ((q, Qo), (k, Ko)):
+        n = onorms.rms_norm(x, w).reshape(1, M, heads, 128)
+        want = orope.rope_apply(n, grid, freq, start) if grid[0] else n
+        assert torch.equal(got.cpu().reshape(1, M, heads, 128), want)
+
+
 def test_rope_identities_on_gpu(gpu):
     """Chunk-offset identity (bit-exact) and norm preservation (tests/test_rope_triton.py:89-104) on the kernel."""
     from wdl import rope

@@ -68,6 +68,12 @@ __device__ __forceinline__ void load8(const uint16_t* p, float* f) {
 // map as one wave over the row. The sum of squares keeps the one-wave order exactly: the first wave's lane sums go
 // through LDS and the second wave continues each from there, value by value, then reduces across lanes. Every load
 // of a wave (its x chunks, norm weights and rotation table entries) is issued before any arithmetic.
+//
+// Bound: Q and K are read and written once, 34 MB at 1392 tokens x 24 heads (7.1 us at the card's copy rate). The
+// rows are short, so what a wave does beside moving them decides: with the table entries loaded and held for each
+// chunk (48 extra registers in fp64) and the grid place from 64-bit divisions it was 12.8 us there (19.6 at 2640
+// tokens, 6.7 at 464); with one set of entries per lane and 32-bit divisions 10.2
+// (15.7 and 5.6).
 template <typename T>
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(NormRopeArgs a) {
     constexpr int CW = MAXCH / 2;  // chunks per lane and wave
@@ -79,8 +85,9 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(NormRopeArgs a) {
               hw = wv % 2;
     const int64_t item = int64_t(blockIdx.x) * 2 + slot;  // (row, which)
     const bool valid = item < a.items * a.M;
-    const int64_t row = valid ? item / a.items : 0;
-    const int which = int(item % a.items);
+    const int pair = a.items - 1;  // items is 1 or 2: a shift and a mask
+    const int64_t row = valid ? item >> pair : 0;
+    const int which = int(item) & pair;
     const uint16_t* src = (which == 0 ? a.q : a.k) + row * (which == 0 ? a.ldq : a.ldk);
     const uint16_t* wt = which == 0 ? a.wq : a.wk;
     uint16_t* dst = (which == 0 ? a.qo : a.ko) + row * a.ldo;
@@ -89,13 +96,36 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(NormRopeArgs a) {
     const int nI = int((chunks + 63) / 64), nI0 = (nI + 1) / 2;
     const int i0 = hw == 0 ? 0 : nI0, i1 = hw == 0 ? nI0 : nI;  // this wave's chunk slots [i0, i1)
     const int64_t hwn = int64_t(a.h) * a.w;
-    const bool rot = row < int64_t(a.f) * hwn;
-    const int pos_t = a.start + int(row / hwn);
-    const int pos_h = int((row / a.w) % a.h);
-    const int pos_w = int(row % a.w);
+    const bool rot = valid && row < int64_t(a.f) * hwn;
+    // a rotated row's place in the grid, in 32 bits (a 64-bit division takes some 150 instructions): f h w <= M, and 2^31
+    // rows of 256 bytes or more exceed the memory. With f = 0 nothing is rotated and h w may be anything: 1 then.
+    const uint32_t r = uint32_t(row), line = r / uint32_t(a.w), frame = r / (rot ? uint32_t(hwn) : 1u);
+    const int pos_t = a.start + int(frame), pos_h = int(line - frame * uint32_t(a.h)),
+              pos_w = int(r - line * uint32_t(a.w));
     constexpr int half = 64, tpairs = half - 2 * (half / 3), spairs = half / 3;  // 22, 21
     uint4 xr[CW], wr[CW];
-    T cs[CW][4], sn[CW][4];
+    // a lane's chunks are 64 chunks = 4 heads apart, so all of them take the table entries of the same 4 pairs p0 .. p0 + 3
+    T cs[4] = {}, sn[4] = {};
+    if (rot) {
+        // one vector load each of cos and sin when the pairs share an axis (all but the two groups that straddle a
+        // boundary)
+        const int p0 = lane * 8 % 128 / 2;
+        const int ax0 = p0 < tpairs ? 0 : (p0 < tpairs + spairs ? 1 : 2);
+        const int ax3 = p0 + 3 < tpairs ? 0 : (p0 + 3 < tpairs + spairs ? 1 : 2);
+        if (a.vec && ax0 == ax3) {
+            const int pos = ax0 == 0 ? pos_t : (ax0 == 1 ? pos_h : pos_w);
+            load4(freq + int64_t(pos) * half + p0, cs);
+            load4(freq + (a.P + pos) * half + p0, sn);
+        } else {
+#pragma unroll
+            for (int p2 = 0; p2 < 4; ++p2) {
+                const int p = p0 + p2;
+                const int pos = p < tpairs ? pos_t : (p < tpairs + spairs ? pos_h : pos_w);
+                cs[p2] = freq[int64_t(pos) * half + p];
+                sn[p2] = freq[(a.P + pos) * half + p];
+            }
+        }
+    }
 #pragma unroll
     for (int k = 0; k < CW; ++k) {
         const int64_t c = lane + 64 * int64_t(i0 + k);
@@ -103,26 +133,6 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(NormRopeArgs a) {
         if (valid && i0 + k < i1 && c < chunks) {
             xr[k] = *reinterpret_cast<const uint4*>(src + c * 8);
             if (wt) wr[k] = *reinterpret_cast<const uint4*>(wt + c * 8);
-            if (rot) {
-                // the chunk's 4 pairs p0 .. p0 + 3: one vector load each of cos and sin when they share an axis
-                // (all but the two groups that straddle an axis boundary)
-                const int p0 = int((c * 8) % 128) / 2;
-                const int ax0 = p0 < tpairs ? 0 : (p0 < tpairs + spairs ? 1 : 2);
-                const int ax3 = p0 + 3 < tpairs ? 0 : (p0 + 3 < tpairs + spairs ? 1 : 2);
-                if (a.vec && ax0 == ax3) {
-                    const int pos = ax0 == 0 ? pos_t : (ax0 == 1 ? pos_h : pos_w);
-                    load4(freq + int64_t(pos) * half + p0, cs[k]);
-                    load4(freq + (a.P + pos) * half + p0, sn[k]);
-                } else {
-#pragma unroll
-                    for (int p2 = 0; p2 < 4; ++p2) {
-                        const int p = p0 + p2;
-                        const int pos = p < tpairs ? pos_t : (p < tpairs + spairs ? pos_h : pos_w);
-                        cs[k][p2] = freq[int64_t(pos) * half + p];
-                        sn[k][p2] = freq[(a.P + pos) * half + p];
-                    }
-                }
-            }
         }
     }
     // sum of squares in the one-wave order: the first wave sums its slots from 0 (absent chunks would add + 0,
@@ -182,8 +192,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(NormRopeArgs a) {
         for (int p2 = 0; p2 < 4; ++p2) {
             if (rot) {
                 const T x1 = T(y[2 * p2]), x2 = T(y[2 * p2 + 1]);
-                o[2 * p2] = f32_to_bf16(float(x1 * cs[k][p2] - x2 * sn[k][p2]));
-                o[2 * p2 + 1] = f32_to_bf16(float(x2 * cs[k][p2] + x1 * sn[k][p2]));
+                o[2 * p2] = f32_to_bf16(float(x1 * cs[p2] - x2 * sn[p2]));
+                o[2 * p2 + 1] = f32_to_bf16(float(x2 * cs[p2] + x1 * sn[p2]));
             } else {
                 o[2 * p2] = f32_to_bf16(y[2 * p2]);
                 o[2 * p2 + 1] = f32_to_bf16(y[2 * p2 + 1]);
