@@ -263,6 +263,36 @@ def test_gemm_split_k_matches_one_pass_and_oracle(gpu, M, N, K, valid):
     assert float((yg.double() - hg).abs().max()) <= 2 ** -7 * float(hg.abs().max()) + 1e-6
 
 
+@pytest.mark.parametrize("M", [1, 31, 33, 77, 128, 129])
+@pytest.mark.parametrize("N,K", [(128, 64), (384, 192), (128, 320), (256, 512), (384, 576), (1536, 1536)])
+def test_gemm_of_few_tokens_equals_the_same_rows_of_a_large_one(gpu, M, N, K):
+    """Few tokens run in 32 x 32 pieces, one wave over all of K, many in 128 x 128 tiles: the same order of the same
+    operations, so bit for bit the same rows, at piece and batch edges (1 to 24 groups) and in every epilogue."""
+    from wdl import ops, w4a4
+
+    g = torch.Generator(device="cuda").manual_seed(M * 31 + N + K)
+    t = w4a4.random_parts(N, K, "cuda", g)
+    wc, ws = ops.as_codes(t["qweight"], K), ops.scale_pairs(t["wscales"])
+    many = 32 * (6 * 256 * 32 // N + 1)
+    x = torch.randn(many, K, device="cuda", generator=g).to(torch.bfloat16)
+    old = torch.randn(many, N, device="cuda", generator=g).to(torch.bfloat16)
+    gate = torch.rand(N, device="cuda", generator=g)
+    for epi in (ops.EPI_BF16, ops.EPI_F32, ops.EPI_RESIDUAL, ops.EPI_GELU):
+        outs, parts = [], []
+        for rows in (M, many):
+            q, a, lora = ops.act_quant_launch(x[:rows], t["smooth"], t["proj_down"])
+            out = old[:rows].float() if epi == ops.EPI_F32 else old[:rows].clone()
+            residual = epi == ops.EPI_RESIDUAL
+            ln = torch.zeros(rows, N // 32, 2, device="cuda") if residual else None
+            ops.gemm_launch(q, a, lora, wc, ws, t["proj_up"], t["bias"], rows, out, epi, gate if residual else None,
+                            stream_k=rows == M, ln_out=ln)
+            outs.append(out)
+            parts.append(ln)
+        assert torch.equal(outs[0], outs[1][:M]), (epi, M, N, K)
+        if parts[0] is not None:
+            assert torch.equal(parts[0], parts[1][:M]), (M, N, K)
+
+
 def test_gemm_residual_and_gelu_epilogues(gpu):
     from wdl import w4a4
 

@@ -1125,6 +1125,101 @@ __global__ __launch_bounds__(512) void w4a4_gemm_bal_kernel(GemmArgs p) {
     gemm_body<128, 128, 64, 64, 4, EPI, STAGES, true, MODE_BAL>(p);
 }
 
+using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
+using u32x2 = uint32_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ auto buffer_of(const void* base, int64_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, uint32_t(bytes), 0x00027000);
+}
+
+// Products of few 32 x 32 pieces (features n0 .., tokens m0 ..): one wave a piece, over all of K in the tiles' order and
+// arithmetic (the same bits as the one-pass launch). Rows past M are left out 32 at a time.
+//
+// Bound by the wave's own instruction stream: it is alone or nearly alone on its SIMD, where each instruction takes 4
+// cycles or more. So the operands come straight into registers through buffer loads (a lane's offset is fixed, a group
+// is one scalar offset: no vector address arithmetic), two batches of FEW_GROUPS groups in turn, and the products of a
+// group run on the matrix core while the previous group's are added. Left to itself the compiler put each product
+// before its own adds and waited for it, with some 40 address instructions a group: 12.5 us for one token at N = K = 3072
+// against 7.2 now; batches of 3 take the same time, of 6 and 8 (twice the registers, one wave a SIMD) up to 1.5 times
+// as long where there are more than 4 pieces a CU.
+constexpr int FEW_GROUPS = 4;
+template <int EPI>
+__global__ __launch_bounds__(64) void w4a4_few_kernel(GemmArgs p, uint32_t rows) {
+    constexpr int PD = FEW_GROUPS;
+    const int lane = threadIdx.x, half = lane / 32;
+    // consecutive pieces, which share a feature slab, on one XCD
+    const uint32_t P = gridDim.x, c = blockIdx.x, pc = P % 8 == 0 ? (c % 8) * (P / 8) + c / 8 : c, slab = pc / rows;
+    const int64_t n0 = int64_t(slab) * 32, m0 = int64_t(pc - slab * rows) * 32;
+    const int G = int(p.K / 64);
+    // the piece's rows of group 0 as buffers (scalar registers), a lane's offsets in them; a group adds a scalar offset
+    const auto wc = buffer_of(p.wc + (n0 / BLOCK_ROWS) * G * BLOCK6 + (n0 % BLOCK_ROWS) * ROW6,
+                              int64_t(G) * BLOCK6 - (n0 % BLOCK_ROWS) * ROW6);
+    const auto qa = buffer_of(p.qa + (m0 / BLOCK_ROWS) * G * BLOCK6 + (m0 % BLOCK_ROWS) * ROW6,
+                              int64_t(G) * BLOCK6 - (m0 % BLOCK_ROWS) * ROW6);
+    const auto ws = buffer_of(p.ws + n0, (G * p.N - n0) * 4);
+    const auto as = buffer_of(p.as + m0, (G * p.Mp - m0) * 2);
+    const int row = lane % 32, o0 = row * ROW6 + 16 * half, o1 = row * ROW6 + 32 + 8 * half;
+    const int wstep = int(p.N * 4), astep = int(p.Mp * 2);
+    const uint32_t low = half == 0 ? ~0u : 0u;
+    struct Batch {
+        u32x6 fa[PD], fb[PD];
+        uint32_t w[PD], a[PD];
+    };
+    Batch b0, b1;
+    auto load = [&](Batch& b, int g) __attribute__((always_inline)) {
+#pragma unroll
+        for (int d = 0; d < PD; ++d) {
+            const uint32_t gg = g + d < G ? g + d : G - 1;  // groups past the last are folded with scales of 0
+            const int at = int(gg * BLOCK6);
+            const u32x4 xa = __builtin_amdgcn_raw_buffer_load_b128(wc, o0, at, 0);
+            const u32x2 ya = __builtin_amdgcn_raw_buffer_load_b64(wc, o1, at, 0);
+            const u32x4 xb = __builtin_amdgcn_raw_buffer_load_b128(qa, o0, at, 0);
+            const u32x2 yb = __builtin_amdgcn_raw_buffer_load_b64(qa, o1, at, 0);
+            b.fa[d] = u32x6{xa[0], xa[1], xa[2], xa[3], ya[0], ya[1]};
+            b.fb[d] = u32x6{xb[0], xb[1], xb[2], xb[3], yb[0], yb[1]};
+            b.w[d] = __builtin_amdgcn_raw_buffer_load_b32(ws, row * 4, int(gg * wstep), 0);
+            b.a[d] = __builtin_amdgcn_raw_buffer_load_b16(as, row * 2, int(gg * astep), 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // the next batch's loads stay behind these (waits are by count)
+    };
+    f32x16 acc[1][1] = {}, I[2], S[2];
+    // group d's fp6 product and the exact product of its scales (lanes 32..63 give the zero k-slots)
+    auto product = [&](const Batch& b, int g, int d, f32x16& x, f32x16& s) __attribute__((always_inline)) {
+        const f32x16 zero = {};
+        const uint32_t keep = g + d < G ? low : 0u;
+        const i16x4 oa = __builtin_bit_cast(i16x4, make_uint2(b.w[d] & keep, 0u));
+        const i16x4 ob = __builtin_bit_cast(i16x4, make_uint2((b.a[d] & keep) * 0x10001u, 0u));
+        const u32x6 ca = b.fa[d], cb = b.fb[d];
+        const i32x8 fa = {int(ca[0]), int(ca[1]), int(ca[2]), int(ca[3]), int(ca[4]), int(ca[5]), 0, 0};
+        const i32x8 fb = {int(cb[0]), int(cb[1]), int(cb[2]), int(cb[3]), int(cb[4]), int(cb[5]), 0, 0};
+        x = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa, fb, zero, 3, 2, 0, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(oa, ob, zero, 0, 0, 0);
+    };
+    auto add = [&](const f32x16& x, const f32x16& s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[0][0][e] = fmaf(x[e], s[e], acc[0][0][e]);
+    };
+    // PD groups: the products of the next group run under the adds of this one
+    auto fold = [&](const Batch& b, int g) __attribute__((always_inline)) {
+        product(b, g, 0, I[0], S[0]);
+#pragma unroll
+        for (int d = 0; d < PD; ++d) {
+            if (d + 1 < PD) product(b, g, d + 1, I[(d + 1) % 2], S[(d + 1) % 2]);
+            __builtin_amdgcn_sched_barrier(0);
+            add(I[d % 2], S[d % 2]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    load(b0, 0);
+    load(b1, PD);
+    for (int g = 0; g < G; g += 2 * PD) {
+        fold(b0, g);
+        load(b0, g + 2 * PD);
+        fold(b1, g + PD);
+        load(b1, g + 3 * PD);
+    }
+    finish_tile<1, 1, EPI>(p, acc, n0, m0, lane);
+}
+
 template <int BN, int BM, int WN, int WM, int NW, int STAGES>
 __global__ __launch_bounds__(NW * 64) void w4a4_gemm_sk_kernel(GemmArgs p) {
     gemm_body<BN, BM, WN, WM, NW, EPI_F32, STAGES, true, MODE_SK>(p);
@@ -1264,8 +1359,36 @@ int64_t sk_shares(int64_t Mp, int64_t N, int64_t K) {
     return 4 * Tw <= 3 * cus ? cus : 0;  // the 256 x 128 launch would leave a quarter of the CUs or more idle
 }
 
+// Few pieces: with 128 x 128 tiles a few tokens give 24 workgroups at N = 3072, each going through K on one CU. Measured
+// (us; tiles -> pieces): N = K = 3072: 1 token 16.7 -> 7.2, 77 17.1 -> 9.3, 464 (5.6 pieces a CU) 17.6 -> 16.0; N =
+// 9216: 128 tokens (4.5) 17.5 -> 13.4, 200 (7.9) 18.1 -> 20.8; N = 16384, K = 512: 33 (4) 6.6 -> 5.5, 77 (6) 6.9 -> 6.9,
+// 128 (8) 7.1 -> 8.7; N = K = 1536: 464 tokens (2.8) 11.0 -> 7.3. Pieces read each operand row once per 32 of the
+// other side, so the tiles win from 6 pieces a CU on. Where stream-K would run, a piece's whole K is the chain: N =
+// 1536, K = 7168: 77 tokens 38.7 -> 13.6, 464 (2.8) 25.3 -> 18.3; N = 3072, K = 8192: 300 (3.8) 28.2 -> 23.4, 464
+// (5.6) 31.7 -> 37.6; K = 14336: 77 29.2 -> 32.4; N = 1024, K = 28672: 42.2 -> 46.1; hence up to K = 128 groups and 3
+// pieces a CU there. A whole captured linear (quantizer and product) of 77 tokens takes 24.4 -> 16.2 us; called one at a
+// time from Python it is bound by the host's 23 us and gains nothing. The buffer offsets are 32 bits wide.
+bool few_fits(int64_t M, int64_t Mp, int64_t N, int64_t K, bool split) {
+    const int64_t cus = cu_count(), G = K / 64, pieces = N / 32 * ((M + 31) / 32);
+    const int64_t most = int64_t(1) << 31;
+    return pieces <= (split ? 3 : 6) * cus && (!split || G <= 128) && G * BLOCK6 < most && G * N * 4 < most &&
+           G * Mp * 2 < most;
+}
+
 int dispatch(const GemmArgs& a, int epi, hipStream_t stream) {
     const int64_t T = (a.N / 128) * (a.Mp / 128), cus = cu_count();
+    const int64_t W = a.part ? sk_shares(a.Mp, a.N, a.K) : 0;
+    if (few_fits(a.M, a.Mp, a.N, a.K, W != 0)) {
+        const uint32_t rows = uint32_t((a.M + 31) / 32), pieces = uint32_t(a.N / 32) * rows;
+        switch (epi) {
+            case EPI_BF16: w4a4_few_kernel<EPI_BF16><<<pieces, 64, 0, stream>>>(a, rows); break;
+            case EPI_F32: w4a4_few_kernel<EPI_F32><<<pieces, 64, 0, stream>>>(a, rows); break;
+            case EPI_RESIDUAL: w4a4_few_kernel<EPI_RESIDUAL><<<pieces, 64, 0, stream>>>(a, rows); break;
+            case EPI_GELU: w4a4_few_kernel<EPI_GELU><<<pieces, 64, 0, stream>>>(a, rows); break;
+            default: return fail(WDL_EINVAL, "w4a4_gemm: bad epilogue %d", epi);
+        }
+        return check_launch("w4a4_gemm few");
+    }
     if (a.part && bal_fits(a.Mp, a.N, a.K)) {
         const unsigned grid = unsigned(cus);
         constexpr int ST = WDL_GEMM_STAGES;
@@ -1278,7 +1401,6 @@ int dispatch(const GemmArgs& a, int epi, hipStream_t stream) {
         }
         return check_launch("w4a4_gemm balanced");
     }
-    const int64_t W = a.part ? sk_shares(a.Mp, a.N, a.K) : 0;
     if (W) {
         const int64_t tiles = (a.N / 256) * (a.Mp / 128);
         w4a4_gemm_sk_kernel<256, 128, 64, 64, SK_NW, WDL_GEMM_STAGES><<<unsigned(W), SK_NW * 64, 0, stream>>>(a);
