@@ -118,12 +118,13 @@ int wdl_w4a4_scale_pairs(const void* scales, int fp16, int64_t n, void* pairs, w
  * Mp % 128 == 0, N % 128 == 0, K % 64 == 0, K <= 2^30; qa, wcodes, out, proj_up, lora, gate and workspace 16-byte
  * aligned, bias 8-byte, scales 4-byte; bf16 outputs: ldo % 8 == 0.
  * workspace: wdl_w4a4_gemm_workspace_bytes(Mp, N, K) bytes (no initial contents), or NULL. When the size is not 0
- * the product runs split in K over one workgroup per CU, for shapes whose tiles leave CUs idle: either the balanced
+ * the product may run split in K over one workgroup per CU, for shapes whose tiles leave CUs idle: either the balanced
  * form (whole tiles dealt evenly, each summed by two halves of K, the few leftover tiles in 32 x 32 pieces summed
  * by eighths of K; one launch, the size is then a 256-byte token the kernel does not touch) or stream-K (the
  * (tile, group) iterations shared evenly, partial sums in the workspace added in a fixed order by a second
- * launch). Both are deterministic, their rounding not identical to the one-pass launch. With NULL the one-pass
- * launch runs. Calls sharing a workspace must not overlap.
+ * launch). Both are deterministic, their rounding not identical to the one-pass launch. With NULL, and for
+ * few tokens (32 x 32 pieces over all of K, the one-pass launch's bits), nothing is split. Calls sharing a workspace
+ * must not overlap.
  * ln_partials (epilogue 2 only, else NULL): fp32 [M][N / 32][2], 16-byte aligned, receives the LayerNorm chunk
  * partials of the rows written (the N columns being whole rows), in wdl_act_quant_w4's order, so the next
  * LayerNorm-fused quantization of out skips its statistics pass. No counterpart in the reference (its LayerNorm

@@ -1,4 +1,5 @@
-"""Loads lib/libwdl.so (the C ABI of include/wdl.h) once through ctypes and raises on any non-zero status.
+"""Loads lib/libwdl.so (the C ABI of include/wdl.h) once through ctypes, and the native launchers over it
+(lib/wdl_host.so), and raises on any non-zero status.
 
 The library is the only compute path: there is no fallback. A missing library raises FileNotFoundError naming the
 build command, as operators.library does for the reference's DLLs (src/wan_dit_lab/kernels/operators.py:12-16).

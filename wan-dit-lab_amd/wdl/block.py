@@ -3,7 +3,7 @@
 WanBlock.forward (src/wan_dit_lab/models/block.py:22-29) with the W4A4 layers installed as the reference's fused
 pack installs them (quantization/w4a4.py:336-352: self_attn.qkv FusedQKVAttention, ffn PackedW4A4GeluMLP, every
 other linear PackedW4A4Linear) and the FP8 KV cache attended through Sage (generation/causal.py:193-210). The
-kernel sequence of one block (about 19 launches, all on the current stream, capturable into one HIP graph):
+kernel sequence of one block (24 launches, all on the current stream, capturable into one HIP graph):
 
   act_quant(X; LN + (1 + scale_a), + shift_a)  -> W4A4 qkv -> norm_rope(q, k) -> kv_append(K, V @ at)
   -> sage_prep(cache[:at] ++ K, V) -> sage_attn (int8 Q quantized in the kernel) -> act_quant(A) -> W4A4 o

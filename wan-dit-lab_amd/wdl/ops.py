@@ -1,7 +1,7 @@
 """The torch operators wdl::* over the C ABI of lib/libwdl.so.
 
 Each operator is a `torch.library.custom_op` whose implementation hands raw device pointers, sizes and the current
-HIP stream to one `wdl_*` launcher, and whose fake (Meta) implementation gives the output shapes, so torch.compile
+HIP stream to one `wdl_*` launcher (the hot ones through the native launchers of host/launch.cpp), and whose fake (Meta) implementation gives the output shapes, so torch.compile
 and graph capture see one opaque op, as the reference's TORCH_LIBRARY ops live::* are
 (native/ops/w4a4_ops.cpp:79-95; native/ops/sage_ops.cpp:28-35). Outputs and workspaces are allocated here, by
 torch, on the current stream; the library allocates nothing.
@@ -351,7 +351,7 @@ def quant_q_launch(x, heads):
 
 
 # token splits of the Sage preparation's column statistics per head (workgroups of colstats_kernel, partials summed in
-# order by finalize_kernel): 16 measured 0.02 ms per step faster than 8 or 32 and 0.14 ms faster than 64
+# order by quant_kv_kernel, finalize_kernel for the statistics alone): 16 measured 0.02 ms per step faster than 8 or 32 and 0.14 ms faster than 64
 SPLITS = 16
 
 
