@@ -299,8 +299,10 @@ int64_t wdl_sage_attn_workspace_bytes(int64_t n, int64_t L, int64_t heads);
  * heads) bytes (no initial contents needed); calls that share a workspace must not overlap. When the (128-query
  * tile, head) pairs just exceed a multiple of the CU count, every CU runs the same number of whole tiles and the
  * key blocks of the remaining tiles are split evenly over half the CUs; their partial softmax states go through the
- * workspace to a second launch that merges them in a fixed order (deterministic). Otherwise the workspace is not
- * touched and may be NULL. */
+ * workspace to a second launch that merges them in a fixed order (deterministic). With at most half as many pairs as
+ * CUs, every tile's key blocks are split in equal shares the same way where that shortens each by 32 blocks of 64
+ * keys or more and a workspace is given
+ * (NULL: whole tiles). Otherwise the workspace is not touched and may be NULL. */
 int wdl_sage_attn(const void* q_i8, int64_t ldq, const float* q_scale, const void* k_i8, const float* k_scale,
                   const void* v_fp8, const float* v_scale, int64_t n, int64_t L, int64_t heads, float sm_scale,
                   void* out, int64_t ldo, void* workspace, wdl_stream_t stream);

@@ -297,6 +297,35 @@ def test_attention_single_key_and_ragged_lengths(gpu):
 
 
 
+@pytest.mark.parametrize("n,L,H", [(1, 2048, 1), (128, 2753, 3), (129, 2816, 2), (464, 4096, 24), (100, 4097, 128),
+                                   (300, 9744, 12), (64, 32768, 1)])
+def test_attention_of_few_tiles_split_over_the_keys(gpu, n, L, H):
+    """Few query tiles over long keys: each tile's keys in shares of 8 blocks or more, merged by a
+    second launch, against whole tiles (no workspace). Either rounds a probability once to e4m3 (relative error 2^-4 at
+    most), so two weighted means of the same values differ by at most 2 * 2^-4 of the largest of them, and a bit. Over
+    values of mixed signs the roundings act as noise of relative rms 2^-4 / sqrt(3) at most in each, independent where the
+    two forms scale a probability differently: 1 - cosine <= 2^-8 / 3."""
+    from wdl import _lib, ops
+
+    g = torch.Generator().manual_seed(n + L + H)
+    K, V = (torch.randn(L, H * 128, generator=g).to(torch.bfloat16).cuda() for _ in range(2))
+    Q = torch.randn(n, H * 128, generator=g).to(torch.bfloat16).cuda()
+    cache = torch.zeros(1, 1, H, 128, dtype=torch.uint8, device="cuda")
+    scale = torch.ones(1, 1, H, 1, device="cuda")
+    prep = ops.sage_prep_launch(cache, scale, cache, scale, K, V, 0)
+    split = ops.sage_attn_q16_launch(Q, prep, L, 128 ** -0.5).float()
+    again = ops.sage_attn_q16_launch(Q, prep, L, 128 ** -0.5).float()
+    whole = _lib.host().sage_attn_q16(Q, prep["k"], prep["k_scale"], prep["v"], prep["v_scale"], L, 128 ** -0.5, None,
+                                      0, None, ops.stream_of(Q)).float()
+    assert torch.equal(split, again)
+    assert (split - whole).abs().max() <= 2.1 * 2 ** -4 * V.float().abs().max()
+    assert osage.cosine(split.cpu(), whole.cpu()) >= 1 - 2 ** -8 / 3
+    exact = torch.nn.functional.scaled_dot_product_attention(
+        *(x.float().cpu().view(-1, H, 128).transpose(0, 1) for x in (Q, K, V))).transpose(0, 1).reshape(n, -1)
+    e_split, e_whole = ((x.cpu() - exact).norm() / exact.norm() for x in (split, whole))
+    assert e_split <= 1.05 * e_whole + 1e-4, (e_split, e_whole)
+
+
 @pytest.mark.parametrize("grid,start,M", [((1, 16, 29), 2, 464), ((3, 16, 29), 0, 1408), ((2, 3, 5), 7, 30)])
 def test_qk_norm_rope_bit_exact(gpu, grid, start, M):
     from wdl import rope

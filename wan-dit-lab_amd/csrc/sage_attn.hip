@@ -129,7 +129,9 @@ __global__ __launch_bounds__(512) void sage_attn_kernel(AttnArgs a) {
     // Work of workgroup w: the whole tiles w, w + W, .. below D (their output written directly), then its share
     // [s0, s1) of the key blocks of the R = T - D remaining tiles, laid end to end (each piece's partial softmax
     // state goes to the workspace slot 2w for its first piece, 2w + 1 for a second; attn_merge_kernel combines them)
-    const int64_t w = blockIdx.x;
+    // With no whole tile (few tiles, every one split) workgroup ids are dealt so that one XCD takes consecutive shares: the
+    // shares of one head read its K / V through one L2.
+    const int64_t w = a.D == 0 && a.W % 8 == 0 ? (blockIdx.x % 8) * (a.W / 8) + blockIdx.x / 8 : blockIdx.x;
     // a dual workgroup: its two groups take whole tiles 2w and 2w + 1 with all the key blocks each, no hand-over
     const bool dualwg = w < a.dual;
     const int64_t T = a.qtiles * a.H, R = T - a.D, Usk = R * nblk;
@@ -576,11 +578,23 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a) {
 }  // namespace
 
 
-// workspace: [2 W][SLOT_FLOATS] fp32 partial states, W <= T (query tiles x heads)
+// Few tiles (at most half the CUs) over long keys: each tile's key blocks in this many equal shares of 8 blocks or more, one
+// workgroup each, where that takes 32 blocks or more off a workgroup's chain (0.57 us each; the partial states and the
+// merge launch cost up to 18 us), 1 for none. Measured (us, whole tiles -> split): 464 queries x 24 heads (96 tiles, 2
+// shares) over 9744 keys 100.1 -> 73.9, over 2784 keys (44 blocks) 38.4 -> 42.5, hence the line; 12 heads (5 shares) over
+// 9744 keys 99.3 -> 44.5; 128 x 24 heads (10) 99.3 -> 34.4; 64 x 12 heads over 4096 keys (8) 46.7 -> 24.3.
+int64_t few_shares(int64_t T, int64_t nblk) {
+    const int64_t cus = cu_count();
+    if (cus <= 0 || cus > MAX_WG || 2 * T > cus) return 1;
+    const int64_t s = cus / T < nblk / 8 ? cus / T : nblk / 8;
+    return s > 1 && nblk - nblk / s >= 32 ? s : 1;
+}
+
+// workspace: [2 W][SLOT_FLOATS] fp32 partial states, W <= T (query tiles x heads) or T few_shares
 extern "C" int64_t wdl_sage_attn_workspace_bytes(int64_t n, int64_t L, int64_t heads) {
     if (n <= 0 || L < 1 || heads <= 0) return 0;
     const int64_t T = (n + 127) / 128 * heads;
-    return 2 * T * SLOT_FLOATS * 4;
+    return 2 * T * few_shares(T, (L + 63) / 64) * SLOT_FLOATS * 4;
 }
 
 static int attn_launch(const void* q_i8, const float* q_scale, const void* q_bf16, int64_t ldq, const void* k_i8,
@@ -611,7 +625,8 @@ static int attn_launch(const void* q_i8, const float* q_scale, const void* q_bf1
     // Short key ranges (no split) with CUs < T <= 2 CUs: one workgroup per CU, and the first T - CUs of them run
     // two whole tiles, one per group of 4 waves over all the key blocks (the other workgroups split their tile's
     // blocks between the groups), so the tiles take one round instead of two.
-    int64_t W = T, Dw = T, dual = 0;
+    // Few tiles over long keys: every tile split (few_shares), where the caller passes a workspace.
+    int64_t W = T, Dw = T, dual = 0, Wt = 0;
     const int64_t cus = cu_count();
     // (under the per-frame mask tiles differ in key count: none is split)
     if (frame == 0 && cus > 0 && cus <= MAX_WG && T > cus && nblk >= 32) {
@@ -620,14 +635,18 @@ static int attn_launch(const void* q_i8, const float* q_scale, const void* q_bf1
         if (T * 100 < 85 * rounds * cus && (cus + 1) * usk < (int64_t(1) << 31)) W = cus, Dw = cus * (T / cus);
     } else if (cus > 0 && T > cus && T <= 2 * cus && (nblk < 32 || cus > MAX_WG)) {
         W = cus, dual = T - cus;
+    } else if (const int64_t s = few_shares(T, nblk);
+               frame == 0 && s > 1 && workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
+        W = Wt = T * s, Dw = 0;
     }
+    if (!Wt) Wt = W / TAIL_DIV > 0 ? W / TAIL_DIV : 1;
     if (Dw < T && (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16))
         return fail(WDL_EINVAL, "sage_attn: a 16-byte aligned workspace of wdl_sage_attn_workspace_bytes is needed");
     float* part = Dw < T ? static_cast<float*>(workspace) : nullptr;
     AttnArgs a{static_cast<const int8_t*>(q_i8), ldq, q_scale, static_cast<const int8_t*>(k_i8), k_scale,
                static_cast<const uint8_t*>(v_fp8), v_scale, static_cast<uint16_t*>(out), ldo, n, L, Lpad, heads,
                sm_scale * 1.4426950408889634f, part, W, qtiles, Dw, static_cast<const uint16_t*>(q_bf16), dual,
-               W / TAIL_DIV > 0 ? W / TAIL_DIV : 1, frame};
+               Wt, frame};
     sage_attn_kernel<<<unsigned(W), 512, 0, stream>>>(a);
     int rc = check_launch("sage_attn");
     if (rc || Dw == T) return rc;

@@ -456,12 +456,25 @@ def reserve(device: torch.device, *, gemm: tuple | None = None, attn: tuple | No
         workspace(_ATTN_WS, device, lib.wdl_sage_attn_workspace_bytes(*(int(v) for v in attn)))
 
 
+def _attn_workspace(n, L, H, device):
+    """The attention's scratch. Calls of few query tiles, which touched none before their keys were split over the idle
+    CUs and may overlap on several streams, get a buffer of their own; the others share the device's."""
+    nbytes = _lib.library().wdl_sage_attn_workspace_bytes(n, L, H)
+    if (n + 127) // 128 * H <= FEW_TILES:
+        return torch.empty(nbytes, device=device, dtype=torch.uint8) if L > 1984 else None  # 31 blocks: never split
+    return workspace(_ATTN_WS, device, nbytes)
+
+
+# query tiles (128 queries of one head) up to which the library may split every tile: half the CUs of an MI355X
+FEW_TILES = 128
+
+
 def sage_attn_launch(q_i8, q_scale, prep, L, sm_scale, out=None):
     """q_i8 [n, H, 128] -> bf16 [n, H*128] (or into `out`, a row-strided [n, H*128] view)."""
     n, H, _ = q_i8.shape
     if out is None:
         out = torch.empty(n, H * 128, device=q_i8.device, dtype=torch.bfloat16)
-    ws = workspace(_ATTN_WS, q_i8.device, _lib.library().wdl_sage_attn_workspace_bytes(n, L, H))
+    ws = _attn_workspace(n, L, H, q_i8.device)
     _lib.call("wdl_sage_attn", ptr(q_i8), H * 128, ptr(q_scale), ptr(prep["k"]), ptr(prep["k_scale"]),
               ptr(prep["v"]), ptr(prep["v_scale"]), n, L, H, float(sm_scale), ptr(out), out.stride(0), ptr(ws),
               stream_of(q_i8))
@@ -482,7 +495,7 @@ def sage_attn_q16_launch(Q, prep, L, sm_scale, out=None, frame_tokens=0):
         if not isinstance(frame_tokens, int) or frame_tokens < 0 or n > L:
             raise ValueError("sage_attn_q16: frame_tokens must be a positive int and the queries among the keys")
     else:
-        ws = workspace(_ATTN_WS, Q.device, _lib.library().wdl_sage_attn_workspace_bytes(n, L, H))
+        ws = _attn_workspace(n, L, H, Q.device)
     return _lib.host().sage_attn_q16(Q, prep["k"], prep["k_scale"], prep["v"], prep["v_scale"], L, sm_scale, out,
                                      int(frame_tokens), ws, stream_of(Q))
 
