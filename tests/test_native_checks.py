@@ -75,3 +75,31 @@ def test_the_native_store_check_passes_only_what_the_check_passes(gpu, at):
         c[name] = BREAKS[how](c[name])
         store = (c["K"], c["V"], c["cache_k"], c["cache_ks"], c["cache_v"], c["cache_vs"], at)
         assert host.kv_valid(*store) == (cache_fp8._refusal(*store) is None), (name, how)
+
+
+FAR = [2 ** 63 - 1, 2 ** 63 - 4, 2 ** 63, 2 ** 64 + 8, -2 ** 63, -2 ** 70]
+
+
+@pytest.mark.parametrize("at", FAR + [9, -1])
+def test_offsets_whose_end_does_not_fit_64_bits_are_refused(at):
+    """at + n beyond int64 is past the cache, not a small negative number, and an offset that no int64 holds is the
+    ValueError of any other offset outside the cache: in the store's and the attention's checks (the store's over
+    tensors that only claim to be on a GPU) and in the C entry, whose pointers are null here."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from wdl import _lib, cache_fp8, sage_kv
+
+    c = _call()
+    with pytest.raises(ValueError, match="at outside the cache"):
+        order = (c["Q"], c["cache_k"], c["cache_ks"], c["cache_v"], c["cache_vs"])
+        sage_kv.attend(*order, at if at != 9 else 13, c["K"], c["V"])
+    with FakeTensorMode():
+        f = {name: torch.empty(t.shape, dtype=t.dtype, device="cuda:0") for name, t in c.items() if name != "at"}
+        store = [f[name] for name in ("K", "V", "cache_k", "cache_ks", "cache_v", "cache_vs")]
+        assert _lib.host().kv_valid(*store, 8) and cache_fp8.refusal(*store, 8) is None
+        kind, message = cache_fp8.refusal(*store, at)
+        assert kind is ValueError and "do not fit a cache of 12 rows" in message
+    if -2 ** 63 <= at < 2 ** 63:
+        lib, strides = _lib.library(), _lib.i64s([1, 1, 1, 1])
+        assert lib.wdl_kv_append_fp8(None, 2, strides, None, 2, strides, 1, 4, 1, 8, None, None, None, None, 12, at, None) == 1
+        assert b"exceeds capacity" in lib.wdl_last_error()

@@ -154,8 +154,9 @@ extern "C" int wdl_kv_append_fp8(const void* k, int k_dtype, const int64_t* k_st
                                  float* cache_ks, void* cache_v, float* cache_vs, int64_t capacity, int64_t at,
                                  hipStream_t stream) {
     if (B < 0 || n < 0 || H < 0 || D < 1) return fail(WDL_EINVAL, "kv_append_fp8: bad shape");
-    if (at < 0 || at + n > capacity) return fail(WDL_EINVAL, "kv_append_fp8: write [%lld, %lld) exceeds capacity %lld",
-                                                 (long long)at, (long long)(at + n), (long long)capacity);
+    if (at < 0 || n > capacity || at > capacity - n)  // (at + n may not fit 64 bits)
+        return fail(WDL_EINVAL, "kv_append_fp8: a write of %lld rows at %lld exceeds capacity %lld", (long long)n,
+                    (long long)at, (long long)capacity);
     if (!k || !v || !cache_k || !cache_ks || !cache_v || !cache_vs || !k_strides || !v_strides)
         return fail(WDL_EINVAL, "kv_append_fp8: null pointer");
     const int64_t rows = B * n * H;

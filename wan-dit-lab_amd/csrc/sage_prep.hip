@@ -532,9 +532,9 @@ extern "C" int wdl_sage_prep_cached_append(void* cache_k, float* cache_ks, void*
                                            float* workspace, void* k_int8, float* k_scale, void* v_fp8,
                                            float* k_mean_out, float* v_scale_out, hipStream_t stream) {
     if (!cache_stats) return fail(WDL_EINVAL, "sage_prep_cached_append: null cache statistics");
-    if (at < 0 || n < 0 || at + n > capacity)
-        return fail(WDL_EINVAL, "sage_prep_cached_append: rows %lld .. %lld outside the cache of %lld", (long long)at,
-                    (long long)(at + n), (long long)capacity);
+    if (at < 0 || n < 0 || n > capacity || at > capacity - n)  // (at + n may not fit 64 bits)
+        return fail(WDL_EINVAL, "sage_prep_cached_append: %lld rows at %lld outside the cache of %lld", (long long)n,
+                    (long long)at, (long long)capacity);
     return sage_prep_launch(cache_k, cache_ks, cache_v, cache_vs, capacity, heads, nullptr, nullptr, k, ldk, v, ldv,
                             heads, at, n, splits, workspace, k_int8, k_scale, v_fp8, k_mean_out, v_scale_out, stream,
                             cache_stats,

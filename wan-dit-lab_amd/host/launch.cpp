@@ -222,7 +222,7 @@ bool kv_valid(const Tensor& k, const Tensor& v, const Tensor& ck, const Tensor& 
         if (t->scalar_type() != at::kFloat || t->dim() != 4 || t->size(0) != ck.size(0) || t->size(1) != ck.size(1) ||
             t->size(2) != ck.size(2) || t->size(3) != 1 || !t->is_contiguous())
             return false;
-    return at >= 0 && at + k.size(1) <= ck.size(1);
+    return at >= 0 && k.size(1) <= ck.size(1) && at <= ck.size(1) - k.size(1);  // (at + n may not fit 64 bits)
 }
 
 // Whether every requirement of sage_kv.py's _check holds for a call without head and token maps

@@ -53,7 +53,7 @@ def _refusal(k, v, cache_k, cache_ks, cache_v, cache_vs, at):
 def refusal(k, v, cache_k, cache_ks, cache_v, cache_vs, at):
     """_refusal, with a call that breaks no requirement passed natively (20 tensor properties in Python took 8 us); a
     compiler traces the Python checks."""
-    if not torch.compiler.is_compiling() and type(at) is int and \
+    if not torch.compiler.is_compiling() and type(at) is int and 0 <= at < 1 << 63 and \
             _lib.host().kv_valid(k, v, cache_k, cache_ks, cache_v, cache_vs, at):
         return None
     return _refusal(k, v, cache_k, cache_ks, cache_v, cache_vs, at)

@@ -64,7 +64,8 @@ def attend(Q, cache_k, cache_ks, cache_v, cache_vs, at, K, V, sm_scale=None, hea
     tokens beside them. append (with cache_stats, not with frame_tokens): K, V also go into cache rows at .. at + n
     (KVCache.store's store_kv_fp8, causal.py:177-181) inside the preparation pass; its requirements are checked
     first, and a broken one raises before anything is written."""
-    if heads is not None or tokens is not None or type(at) is not int or torch.compiler.is_compiling() or \
+    if heads is not None or tokens is not None or torch.compiler.is_compiling() or type(at) is not int or \
+            not 0 <= at < 1 << 63 or \
             not _lib.host().attend_valid(Q, cache_k, cache_ks, cache_v, cache_vs, at, K, V):
         _check(Q, cache_k, cache_ks, cache_v, cache_vs, at, K, V, heads, tokens)
     if append:
