@@ -290,7 +290,13 @@ int wdl_sage_prep_cached_append(void* cache_k, float* cache_ks, void* cache_v, f
 int wdl_sage_sm89_relayout(const void* k_i8, int64_t ldk, const void* v_fp8, int64_t v_stride_d, int64_t v_stride_h,
                            int64_t L, int64_t heads, void* k_out, void* v_out, wdl_stream_t stream);
 
-/* Workspace (bytes) of wdl_sage_attn for n queries, L keys and `heads` heads. */
+/* How wdl_sage_attn and wdl_sage_attn_q16 run n queries over L keys when they are given a workspace: 0 every (128-query
+ * tile, head) whole (the workspace is not touched and may be NULL), 1 the tiles past the last whole round over the CUs
+ * split (a workspace is needed), s >= 2 every tile's keys in s equal shares (NULL: whole tiles). */
+int wdl_sage_attn_split(int64_t n, int64_t L, int64_t heads);
+
+/* Workspace (bytes) of wdl_sage_attn for n queries and `heads` heads. The same for every L, and never less for more
+ * queries or heads: a buffer of the size for a program's largest call serves its smaller ones. */
 int64_t wdl_sage_attn_workspace_bytes(int64_t n, int64_t L, int64_t heads);
 
 /* Sage-2 style attention (int8 QK^T, fp32 online softmax, fp8 PV, non-causal). Replaces live::sage_sm89
@@ -301,8 +307,8 @@ int64_t wdl_sage_attn_workspace_bytes(int64_t n, int64_t L, int64_t heads);
  * key blocks of the remaining tiles are split evenly over half the CUs; their partial softmax states go through the
  * workspace to a second launch that merges them in a fixed order (deterministic). With at most half as many pairs as
  * CUs, every tile's key blocks are split in equal shares the same way where that shortens each by 32 blocks of 64
- * keys or more and a workspace is given
- * (NULL: whole tiles). Otherwise the workspace is not touched and may be NULL. */
+ * keys or more and a workspace is given (NULL: whole tiles). Otherwise the workspace is not touched and may be NULL
+ * (wdl_sage_attn_split says which). */
 int wdl_sage_attn(const void* q_i8, int64_t ldq, const float* q_scale, const void* k_i8, const float* k_scale,
                   const void* v_fp8, const float* v_scale, int64_t n, int64_t L, int64_t heads, float sm_scale,
                   void* out, int64_t ldo, void* workspace, wdl_stream_t stream);

@@ -297,6 +297,33 @@ def test_attention_single_key_and_ragged_lengths(gpu):
 
 
 
+def test_a_workspace_sized_for_the_largest_call_serves_every_smaller_one(gpu):
+    """A program may size one attention workspace for its longest chunk, and before its window has filled: the size
+    does not depend on the keys, never falls as queries or heads grow, and covers the two slots a workgroup that any
+    smaller call splits over may write (wdl_sage_attn_split; the launch is not run)."""
+    from wdl import _lib
+
+    lib = _lib.library()
+    slot = 4 * 4 * (64 * 64 + 128)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    kinds = set()
+    for n in (1, 128, 129, 464, 640, 1392, 1408, 2640, 5280):
+        for H in (1, 5, 12, 24, 40):
+            tiles = (n + 127) // 128 * H
+            sizes = {lib.wdl_sage_attn_workspace_bytes(n, L, H) for L in (1, 2048, 2753, 9744, 32768)}
+            assert len(sizes) == 1
+            assert all(lib.wdl_sage_attn_workspace_bytes(m, 9744, h) <= max(sizes) for m in (1, n // 2 + 1, n) for h in
+                       (1, H // 2 + 1, H))
+            for L in (1, 2048, 2753, 9744, 32768):
+                split = lib.wdl_sage_attn_split(n, L, H)
+                kinds.add(min(split, 2))
+                assert split == 0 or split == 1 and tiles > cus or split >= 2 and tiles * split <= cus
+                groups = {0: 0, 1: cus}.get(split, tiles * split)
+                assert 2 * groups * slot <= max(sizes), (n, H, L, split)
+    assert kinds == {0, 1, 2}
+    assert lib.wdl_sage_attn_workspace_bytes(0, 64, 24) == lib.wdl_sage_attn_split(0, 64, 24) == 0
+
+
 @pytest.mark.parametrize("n,L,H", [(1, 2048, 1), (128, 2753, 3), (129, 2816, 2), (464, 4096, 24), (100, 4097, 128),
                                    (300, 9744, 12), (64, 32768, 1)])
 def test_attention_of_few_tiles_split_over_the_keys(gpu, n, L, H):

@@ -575,9 +575,6 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a) {
         make_uint2(rr[0] | (uint32_t(rr[1]) << 16), rr[2] | (uint32_t(rr[3]) << 16));
 }
 
-}  // namespace
-
-
 // Few tiles (at most half the CUs) over long keys: each tile's key blocks in this many equal shares of 8 blocks or more, one
 // workgroup each, where that takes 32 blocks or more off a workgroup's chain (0.57 us each; the partial states and the
 // merge launch cost up to 18 us), 1 for none. Measured (us, whole tiles -> split): 464 queries x 24 heads (96 tiles, 2
@@ -590,11 +587,52 @@ int64_t few_shares(int64_t T, int64_t nblk) {
     return s > 1 && nblk - nblk / s >= 32 ? s : 1;
 }
 
-// workspace: [2 W][SLOT_FLOATS] fp32 partial states, W <= T (query tiles x heads) or T few_shares
-extern "C" int64_t wdl_sage_attn_workspace_bytes(int64_t n, int64_t L, int64_t heads) {
+// How the T = (query tiles) x (heads) tiles over nblk key blocks run: on W workgroups, the first D tiles whole (D of
+// AttnArgs), the key blocks of the others over the first Wt workgroups.
+// One workgroup per tile, unless that leaves a large share of the last round of CUs idle (tiles just above a
+// multiple of the CU count): then one workgroup per CU runs floor(T / CUs) whole tiles each and the key blocks
+// of the T mod CUs remaining tiles are split evenly over half of them, merged by a second launch. Short key
+// ranges keep one workgroup per tile.
+// Short key ranges (no split) with CUs < T <= 2 CUs: one workgroup per CU, and the first T - CUs of them run
+// two whole tiles, one per group of 4 waves over all the key blocks (the other workgroups split their tile's
+// blocks between the groups), so the tiles take one round instead of two.
+// Few tiles over long keys: every tile split (few_shares), where the caller passes a workspace.
+// Under the per-frame mask tiles differ in key count: none is split.
+struct Split {
+    int64_t W, D, dual, Wt;
+};
+Split split_of(int64_t T, int64_t nblk, int64_t frame, bool workspace) {
+    Split s{T, T, 0, 0};
+    const int64_t cus = cu_count();
+    if (frame == 0 && cus > 0 && cus <= MAX_WG && T > cus && nblk >= 32) {
+        const int64_t rounds = (T + cus - 1) / cus;
+        const int64_t usk = (T % cus) * nblk;  // key blocks of the split tiles
+        if (T * 100 < 85 * rounds * cus && (cus + 1) * usk < (int64_t(1) << 31)) s.W = cus, s.D = cus * (T / cus);
+    } else if (cus > 0 && T > cus && T <= 2 * cus && (nblk < 32 || cus > MAX_WG)) {
+        s.W = cus, s.dual = T - cus;
+    } else if (const int64_t shares = few_shares(T, nblk); frame == 0 && shares > 1 && workspace) {
+        s.W = s.Wt = T * shares, s.D = 0;
+    }
+    if (!s.Wt) s.Wt = s.W / TAIL_DIV > 0 ? s.W / TAIL_DIV : 1;
+    return s;
+}
+
+}  // namespace
+
+extern "C" int wdl_sage_attn_split(int64_t n, int64_t L, int64_t heads) {
     if (n <= 0 || L < 1 || heads <= 0) return 0;
     const int64_t T = (n + 127) / 128 * heads;
-    return 2 * T * few_shares(T, (L + 63) / 64) * SLOT_FLOATS * 4;
+    const Split s = split_of(T, (L + 63) / 64, 0, true);
+    return s.D == T ? 0 : s.D > 0 ? 1 : int(s.W / T);
+}
+
+// [2 W][SLOT_FLOATS] fp32 partial states. A split launch has at most T workgroups when it splits leftover tiles, and at
+// most one per CU when it splits few tiles, for any L: a buffer sized for the largest call then serves every smaller one
+// (sized by few_shares(T) it was larger for 24 tiles of ten shares than for 130 tiles).
+extern "C" int64_t wdl_sage_attn_workspace_bytes(int64_t n, int64_t L, int64_t heads) {
+    if (n <= 0 || L < 1 || heads <= 0) return 0;
+    const int64_t T = (n + 127) / 128 * heads, cus = cu_count(), few = cus <= MAX_WG ? cus : 0;
+    return 2 * (T > few ? T : few) * SLOT_FLOATS * 4;
 }
 
 static int attn_launch(const void* q_i8, const float* q_scale, const void* q_bf16, int64_t ldq, const void* k_i8,
@@ -618,35 +656,15 @@ static int attn_launch(const void* q_i8, const float* q_scale, const void* q_bf1
     if ((reinterpret_cast<uintptr_t>(k_i8) | reinterpret_cast<uintptr_t>(v_fp8)) % 16)
         return fail(WDL_EINVAL, "sage_attn: K / V must be 16-byte aligned");
     const int64_t qtiles = (n + 127) / 128, T = qtiles * heads, nblk = Lpad / 64;
-    // One workgroup per tile, unless that leaves a large share of the last round of CUs idle (tiles just above a
-    // multiple of the CU count): then one workgroup per CU runs floor(T / CUs) whole tiles each and the key blocks
-    // of the T mod CUs remaining tiles are split evenly over all of them, merged by a second launch. Short key
-    // ranges keep one workgroup per tile.
-    // Short key ranges (no split) with CUs < T <= 2 CUs: one workgroup per CU, and the first T - CUs of them run
-    // two whole tiles, one per group of 4 waves over all the key blocks (the other workgroups split their tile's
-    // blocks between the groups), so the tiles take one round instead of two.
-    // Few tiles over long keys: every tile split (few_shares), where the caller passes a workspace.
-    int64_t W = T, Dw = T, dual = 0, Wt = 0;
-    const int64_t cus = cu_count();
-    // (under the per-frame mask tiles differ in key count: none is split)
-    if (frame == 0 && cus > 0 && cus <= MAX_WG && T > cus && nblk >= 32) {
-        const int64_t rounds = (T + cus - 1) / cus;
-        const int64_t usk = (T % cus) * nblk;  // key blocks of the split tiles
-        if (T * 100 < 85 * rounds * cus && (cus + 1) * usk < (int64_t(1) << 31)) W = cus, Dw = cus * (T / cus);
-    } else if (cus > 0 && T > cus && T <= 2 * cus && (nblk < 32 || cus > MAX_WG)) {
-        W = cus, dual = T - cus;
-    } else if (const int64_t s = few_shares(T, nblk);
-               frame == 0 && s > 1 && workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
-        W = Wt = T * s, Dw = 0;
-    }
-    if (!Wt) Wt = W / TAIL_DIV > 0 ? W / TAIL_DIV : 1;
+    const Split s = split_of(T, nblk, frame, workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0);
+    const int64_t W = s.W, Dw = s.D;
     if (Dw < T && (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16))
         return fail(WDL_EINVAL, "sage_attn: a 16-byte aligned workspace of wdl_sage_attn_workspace_bytes is needed");
     float* part = Dw < T ? static_cast<float*>(workspace) : nullptr;
     AttnArgs a{static_cast<const int8_t*>(q_i8), ldq, q_scale, static_cast<const int8_t*>(k_i8), k_scale,
                static_cast<const uint8_t*>(v_fp8), v_scale, static_cast<uint16_t*>(out), ldo, n, L, Lpad, heads,
-               sm_scale * 1.4426950408889634f, part, W, qtiles, Dw, static_cast<const uint16_t*>(q_bf16), dual,
-               Wt, frame};
+               sm_scale * 1.4426950408889634f, part, W, qtiles, Dw, static_cast<const uint16_t*>(q_bf16), s.dual,
+               s.Wt, frame};
     sage_attn_kernel<<<unsigned(W), 512, 0, stream>>>(a);
     int rc = check_launch("sage_attn");
     if (rc || Dw == T) return rc;

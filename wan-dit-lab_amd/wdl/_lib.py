@@ -62,6 +62,7 @@ SIGNATURES: dict[str, list] = {
     "wdl_sage_prep_cached_append": [c_ptr, c_ptr, c_ptr, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_i64, c_i64,
                                     c_i64, c_ptr, c_int, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr],
     "wdl_sage_sm89_relayout": [c_ptr, c_i64, c_ptr, c_i64, c_i64, c_i64, c_i64, c_ptr, c_ptr, c_ptr],
+    "wdl_sage_attn_split": [c_i64, c_i64, c_i64],
     "wdl_sage_attn_workspace_bytes": [c_i64, c_i64, c_i64],
     "wdl_sage_attn": [c_ptr, c_i64, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_i64, c_i64, c_i64, c_f32, c_ptr, c_i64,
                       c_ptr, c_ptr],

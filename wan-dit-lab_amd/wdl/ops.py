@@ -457,16 +457,14 @@ def reserve(device: torch.device, *, gemm: tuple | None = None, attn: tuple | No
 
 
 def _attn_workspace(n, L, H, device):
-    """The attention's scratch. Calls of few query tiles, which touched none before their keys were split over the idle
-    CUs and may overlap on several streams, get a buffer of their own; the others share the device's."""
-    nbytes = _lib.library().wdl_sage_attn_workspace_bytes(n, L, H)
-    if (n + 127) // 128 * H <= FEW_TILES:
-        return torch.empty(nbytes, device=device, dtype=torch.uint8) if L > 1984 else None  # 31 blocks: never split
-    return workspace(_ATTN_WS, device, nbytes)
-
-
-# query tiles (128 queries of one head) up to which the library may split every tile: half the CUs of an MI355X
-FEW_TILES = 128
+    """The attention's scratch, None where every tile runs whole. Calls of few query tiles, all of them split, touched
+    none before and may overlap on several streams, so each gets a buffer of its own; the others share the device's."""
+    lib = _lib.library()
+    split = lib.wdl_sage_attn_split(n, L, H)
+    if not split:
+        return None
+    nbytes = lib.wdl_sage_attn_workspace_bytes(n, L, H)
+    return torch.empty(nbytes, device=device, dtype=torch.uint8) if split > 1 else workspace(_ATTN_WS, device, nbytes)
 
 
 def sage_attn_launch(q_i8, q_scale, prep, L, sm_scale, out=None):
