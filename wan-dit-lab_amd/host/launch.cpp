@@ -255,18 +255,20 @@ PYBIND11_MODULE(wdl_host, m) {
         }
     });
     m.def("bind", &bind);
-    m.def("act_quant", &act_quant);
-    m.def("gemm", &gemm);
-    m.def("gelu_quant", &gelu_quant);
-    m.def("qk_norm_rope", &qk_norm_rope);
-    m.def("sage_prep", &sage_prep);
-    m.def("sage_attn_q16", &sage_attn_q16);
-    m.def("attn_bf16", &attn_bf16);
-    m.def("kv_append", &kv_append);
-    m.def("fp8_quantize", &fp8_quantize);
-    m.def("fp8_gemm", &fp8_gemm);
-    m.def("fp8wo_gemm", &fp8wo_gemm);
-    m.def("rope3d", &rope3d);
+    // an allocation or a launch may wait (allocator retry, first module load, full queue): other Python threads run on
+    const py::call_guard<py::gil_scoped_release> nogil;
+    m.def("act_quant", &act_quant, nogil);
+    m.def("gemm", &gemm, nogil);
+    m.def("gelu_quant", &gelu_quant, nogil);
+    m.def("qk_norm_rope", &qk_norm_rope, nogil);
+    m.def("sage_prep", &sage_prep, nogil);
+    m.def("sage_attn_q16", &sage_attn_q16, nogil);
+    m.def("attn_bf16", &attn_bf16, nogil);
+    m.def("kv_append", &kv_append, nogil);
+    m.def("fp8_quantize", &fp8_quantize, nogil);
+    m.def("fp8_gemm", &fp8_gemm, nogil);
+    m.def("fp8wo_gemm", &fp8wo_gemm, nogil);
+    m.def("rope3d", &rope3d, nogil);
     m.def("kv_valid", &kv_valid);
     m.def("attend_valid", &attend_valid);
 }
