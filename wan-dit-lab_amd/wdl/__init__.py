@@ -10,6 +10,10 @@ __all__ = ["build"]
 
 
 def build(force: bool = False):
+    """Compiles the library and the native launchers over it (both are needed); returns the library's path."""
     from wdl.build import build as _build
+    from wdl.build import build_host
 
-    return _build(force=force)
+    lib = _build(force=force)
+    build_host(force=force)
+    return lib

@@ -1,4 +1,5 @@
-"""Builds the C-ABI library lib/libwdl.so from csrc/*.hip with hipcc for gfx950 only.
+"""Builds the C-ABI library lib/libwdl.so from csrc/*.hip with hipcc for gfx950 only (build), and the native
+launchers lib/wdl_host.so from host/launch.cpp with g++ (build_host).
 
 Each source compiles to its own object in parallel (`hipcc -c`), then one `hipcc -shared` link. Flags:
 - `-ffp-contract=off`: no implicit fused multiply-adds, so every kernel rounds exactly as its source is written
@@ -6,7 +7,7 @@ Each source compiles to its own object in parallel (`hipcc -c`), then one `hipcc
 - `-Xclang -target-feature -Xclang -packed-fp32-ops`: no packed FP32 VALU instructions are generated;
 - `-munsafe-fp-atomics` is NOT used: the library has no floating-point atomics.
 
-Run as `python -m wdl.build` from the package root, or call build().
+Run as `python -m wdl.build` from the package root, or call wdl.build().
 """
 
 from __future__ import annotations
@@ -23,6 +24,7 @@ OBJ = ROOT / "_build"
 LIB = ROOT / "lib" / "libwdl.so"
 HOST_SRC = ROOT / "host" / "launch.cpp"
 HOST = ROOT / "lib" / "wdl_host.so"
+HEADER = ROOT.parent / "include" / "wdl.h"
 ARCH = "gfx950"
 
 FLAGS = [
@@ -76,8 +78,11 @@ def build(force: bool = False, jobs: int | None = None) -> Path:
     return LIB
 
 
-def build_host() -> Path:
-    """Compiles the native launchers (host/launch.cpp, against torch's headers) into lib/wdl_host.so."""
+def build_host(force: bool = False) -> Path:
+    """Compiles the native launchers (host/launch.cpp, against torch's headers) into lib/wdl_host.so, unless that is
+    newer than they and the C ABI's header."""
+    if not force and HOST.exists() and all(HOST.stat().st_mtime >= d.stat().st_mtime for d in (HOST_SRC, HEADER)):
+        return HOST
     import sysconfig
 
     import torch
@@ -85,7 +90,7 @@ def build_host() -> Path:
 
     HOST.parent.mkdir(exist_ok=True)
     tmp = HOST.with_suffix(".so.tmp")
-    includes = [str(ROOT.parent / "include"), *cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
+    includes = [str(HEADER.parent), *cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
     cmd = ["g++", "-O2", "-std=c++17", "-shared", "-fPIC", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            "-DTORCH_EXTENSION_NAME=wdl_host", *(f for i in includes for f in ("-isystem", i)), str(HOST_SRC), "-o", str(tmp),
            *(f"-L{p}" for p in cpp_extension.library_paths()), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
@@ -98,4 +103,4 @@ def build_host() -> Path:
 
 if __name__ == "__main__":
     print(build(force="--force" in sys.argv))
-    print(build_host())
+    print(build_host(force="--force" in sys.argv))
