@@ -27,7 +27,9 @@ typedef void* wdl_stream_t; /* a hipStream_t */
 
 /* Message of the last failed call on this host thread ("" after a success). */
 const char* wdl_last_error(void);
+/* The version of this interface that the library implements: WDL_ABI_VERSION where both are of one build. */
 int wdl_abi_version(void);
+#define WDL_ABI_VERSION 14
 
 /* FP8 KV-cache append. Replaces store_kv_fp8 / wan_dit_lab::store_kv_fp8_<hash>
  * (src/wan_dit_lab/kernels/cache_fp8.py:59-72, 75-105) and KVCache.store's fp8 branch

@@ -16,7 +16,7 @@ for p in (ROOT / "wan-dit-lab_amd", ROOT):
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs an MI355X (gfx950) and lib/libwdl.so")
+    config.addinivalue_line("markers", "gpu: needs an MI355X (gfx950), lib/libwdl.so and lib/wdl_host.so")
     config.addinivalue_line("markers", "slow: long-running")
 
 
@@ -28,5 +28,5 @@ def gpu():
         pytest.skip("GPU required")
     from wdl import _lib
 
-    _lib.library()  # raises FileNotFoundError when the library is not built
+    _lib.host()  # raises FileNotFoundError when the library or its native launchers are not built
     return torch.device("cuda:0")

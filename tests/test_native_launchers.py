@@ -15,13 +15,11 @@ SLEEP = 0.2
 BF = torch.bfloat16
 
 
-@pytest.fixture(scope="module")
-def stand_in(tmp_path_factory):
-    """A copy of the launchers (entry points of its own) bound to the stand-in."""
+def _stand_in(at, version):
+    """A copy of the launchers, whose entry points are its own, and a stand-in of that ABI version."""
     from wdl import _lib
 
     _lib.host()  # built and loadable
-    at = tmp_path_factory.mktemp("stand_in")
     lines = ["#include <unistd.h>"]
     for name in _lib.SIGNATURES:
         if name == "wdl_last_error":
@@ -29,7 +27,7 @@ def stand_in(tmp_path_factory):
         elif _lib.RESTYPES.get(name) is _lib.c_i64:
             lines.append(f"long {name}() {{ return 64; }}")
         elif name == "wdl_abi_version":
-            lines.append(f"int {name}() {{ return {_lib.library().wdl_abi_version()}; }}")
+            lines.append(f"int {name}() {{ return {version}; }}")
         else:
             lines.append(f"int {name}() {{ usleep({int(SLEEP * 1e6)}); return 0; }}")
     (at / "stub.c").write_text("\n".join(lines))
@@ -38,8 +36,28 @@ def stand_in(tmp_path_factory):
     loader = importlib.machinery.ExtensionFileLoader("wdl_host", str(at / "wdl_host.so"))
     module = importlib.util.module_from_spec(importlib.util.spec_from_loader("wdl_host", loader))
     loader.exec_module(module)
-    module.bind(str(at / "stub.so"))
+    return module, str(at / "stub.so")
+
+
+@pytest.fixture(scope="module")
+def stand_in(tmp_path_factory):
+    from wdl import _lib
+
+    module, library = _stand_in(tmp_path_factory.mktemp("stand_in"), _lib.library().wdl_abi_version())
+    module.bind(library)
     return module
+
+
+def test_a_library_of_another_abi_version_is_refused(tmp_path):
+    """The launchers pass the arguments of the header they were compiled with: beside a library of another version they
+    would pass wrong ones, so binding refuses it and names both."""
+    from wdl import _lib
+
+    version = _lib.library().wdl_abi_version()
+    assert f"#define WDL_ABI_VERSION {version}\n" in (_lib.LIB_PATH.parents[2] / "include" / "wdl.h").read_text()
+    module, library = _stand_in(tmp_path, version + 1)
+    with pytest.raises(RuntimeError, match=f"ABI version {version + 1}, .* compiled for {version}"):
+        module.bind(library)
 
 
 def _calls():

@@ -20,7 +20,8 @@ using at::Tensor;
 using Opt = std::optional<Tensor>;
 
 #define WDL_ENTRIES(X)                                                                                              \
-    X(wdl_last_error) X(wdl_kv_append_fp8) X(wdl_act_quant_workspace_floats) X(wdl_act_quant_w4) X(wdl_w4a4_gemm)   \
+    X(wdl_last_error) X(wdl_abi_version) X(wdl_kv_append_fp8) X(wdl_act_quant_workspace_floats) X(wdl_act_quant_w4) \
+    X(wdl_w4a4_gemm)                                                                                                \
     X(wdl_w4a4_gemm_gelu_quant_workspace_floats) X(wdl_w4a4_gemm_gelu_quant) X(wdl_fp8_quantize_workspace_floats)   \
     X(wdl_fp8_quantize) X(wdl_fp8_gemm) X(wdl_fp8wo_gemm) X(wdl_qk_norm_rope) X(wdl_sage_prep_workspace_floats)     \
     X(wdl_sage_prep) X(wdl_sage_prep_cached) X(wdl_sage_prep_cached_append) X(wdl_sage_attn_q16)                    \
@@ -41,6 +42,10 @@ void bind(const std::string& path) {
     if (!e.name) throw std::runtime_error(path + " has no entry point " #name);
     WDL_ENTRIES(X)
 #undef X
+    if (e.wdl_abi_version() != WDL_ABI_VERSION)
+        throw std::runtime_error(path + " has ABI version " + std::to_string(e.wdl_abi_version()) +
+                                 ", the launchers are compiled for " + std::to_string(WDL_ABI_VERSION) +
+                                 ": build both again (python -m wdl.build)");
     lib = e;
 }
 
