@@ -104,3 +104,32 @@ def test_other_threads_run_while_a_launch_waits(stand_in, name):
         ticks += 1
     launch.join()
     assert ticks >= 10, ticks
+
+
+@pytest.mark.parametrize("name,which,more", [("act_quant", 0, 1), ("act_quant", 0, -1), ("qk_norm_rope", 0, 1),
+                                             ("qk_norm_rope", 0, -1), ("kv_append", 0, 1), ("kv_append", 0, -1),
+                                             ("kv_append", 1, -1), ("rope3d", 0, 1), ("rope3d", 0, -1),
+                                             ("rope3d", 1, -1)])
+def test_tensors_of_another_number_of_dimensions_are_refused(stand_in, name, which, more):
+    """The operators under the checked functions read sizes and strides by position: a tensor with a dimension too
+    many would be read as if its last one were not there."""
+    args = list(_calls()[name])
+    args[which] = args[which][..., None] if more > 0 else args[which][0]
+    with pytest.raises(ValueError, match="dimensions"):
+        getattr(stand_in, name)(*args)
+
+
+def test_the_rotation_needs_a_grid_for_each_sample(stand_in):
+    args = list(_calls()["rope3d"])
+    args[2] = [1, 2]
+    with pytest.raises(ValueError, match="grid"):
+        stand_in.rope3d(*args)
+
+
+@pytest.mark.parametrize("shape,key", [((0, 4, 2, 128), ""), ((1, 0, 2, 128), "0,1,1"), ((0, 0, 2, 128), "1,1,1")])
+def test_an_empty_rotation_needs_no_launch(shape, key):
+    """The operator gives an empty tensor for an empty one, whatever the grids, also where there is no GPU."""
+    import wdl.rope
+
+    y = wdl.rope.rope3d_rotate(torch.empty(shape), torch.zeros(2, 16, 64), key, 0, False, BF)
+    assert y.shape == shape and y.dtype == BF

@@ -73,12 +73,20 @@ int code(at::ScalarType t) {
     }
 }
 
+// sizes and strides below are read by position
+void dims(const char* what, const Tensor& t, int64_t least, int64_t most) {
+    if (t.dim() < least || t.dim() > most)
+        throw std::invalid_argument(std::string(what) + ": a tensor of " + std::to_string(t.dim()) + " dimensions, not " +
+                                    std::to_string(least));
+}
+
 constexpr int64_t PAD = 128, ROW6 = 48, RANK = 32, D = 128;
 
 std::tuple<Tensor, Tensor, Opt> act_quant(const Tensor& x, const Tensor& smooth, const Opt& pdt, double qshift,
                                           bool is_unsigned, bool ln, const Opt& shift, const Opt& scale,
                                           const Opt& weight, const Opt& bias, double eps, const Opt& partials,
                                           const Opt& v_out, uintptr_t stream) {
+    dims("act_quant x", x, 2, 2);
     const int64_t M = x.size(0), K = x.size(1), Mp = (M + PAD - 1) / PAD * PAD;
     Tensor q = buf(x, {Mp / PAD, K / 64, PAD, ROW6}, at::kByte), asc = buf(x, {K / 64, Mp}, at::kBFloat16);
     Opt lora;
@@ -113,6 +121,7 @@ std::tuple<Tensor, Tensor, Tensor> gelu_quant(const Tensor& q, const Tensor& asc
 std::tuple<Tensor, Opt> qk_norm_rope(const Tensor& q, const Opt& k, const Opt& wq, const Opt& wk, const Tensor& freq,
                                      int f, int h, int w, int64_t start, double eps, const Opt& q_into,
                                      const Opt& k_into, uintptr_t stream) {
+    dims("qk_norm_rope q", q, 2, 2);
     const int64_t M = q.size(0), C = q.size(1);
     Tensor qo = q_into ? *q_into : buf(q, {M, C}, at::kBFloat16);
     Opt ko = k_into;
@@ -168,6 +177,8 @@ Tensor attn_bf16(const Tensor& q, const Tensor& kp, const Tensor& vp, int64_t L,
 
 void kv_append(const Tensor& k, const Tensor& v, const Tensor& ck, const Tensor& cks, const Tensor& cv,
                const Tensor& cvs, int64_t at, uintptr_t stream) {
+    dims("kv_append k", k, 4, 4);
+    dims("kv_append v", v, 4, 64);
     CALL(wdl_kv_append_fp8, ptr(k), code(k.scalar_type()), k.strides().data(), ptr(v), code(v.scalar_type()),
          v.strides().data(), k.size(0), k.size(1), k.size(2), k.size(3), ptr(ck), f32(cks), ptr(cv), f32(cvs), ck.size(1),
          at, str(stream));
@@ -201,11 +212,13 @@ void fp8wo_gemm(const Tensor& x, const Tensor& w, const Tensor& ws, const Opt& b
 
 Tensor rope3d(const Tensor& x, const Tensor& freq, const std::vector<int32_t>& grids, int64_t start, bool inverse,
               at::ScalarType type, uintptr_t stream) {
+    dims("rope3d x", x, 4, 4);
+    dims("rope3d freq", freq, 3, 64);
+    if (int64_t(grids.size()) < 3 * x.size(0)) throw std::invalid_argument("rope3d: one grid of 3 sizes per sample");
     Tensor out = buf(x, x.sizes(), type);
-    if (x.numel())
-        CALL(wdl_rope3d_rotate, ptr(x), code(x.scalar_type()), x.strides().data(), ptr(freq), code(freq.scalar_type()),
-             freq.strides().data(), freq.size(1), x.size(0), x.size(1), x.size(2), x.size(3), grids.data(), start, inverse,
-             ptr(out), code(type), str(stream));
+    CALL(wdl_rope3d_rotate, ptr(x), code(x.scalar_type()), x.strides().data(), ptr(freq), code(freq.scalar_type()),
+         freq.strides().data(), freq.size(1), x.size(0), x.size(1), x.size(2), x.size(3), grids.data(), start, inverse,
+         ptr(out), code(type), str(stream));
     return out;
 }
 

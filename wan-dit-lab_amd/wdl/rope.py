@@ -63,6 +63,8 @@ def rope3d_rotate(x: torch.Tensor, freq: torch.Tensor, grid_key: str, start: int
     """wan_dit_lab::rope3d_rotate (kernels/rope_triton.py:66-81) on wdl_rope3d_rotate: x [B, L, H, dim] (any strides)
     turned by the 3D RoPE angles of the grids in grid_key ("f,h,w,f,h,w,..."), by -angle when inverse; a new
     contiguous tensor of output_dtype."""
+    if not x.numel():
+        return torch.empty(x.shape, device=x.device, dtype=output_dtype)
     return _lib.host().rope3d(x, freq, [int(v) for v in grid_key.split(",")], start, inverse, output_dtype, stream_of(x))
 
 
