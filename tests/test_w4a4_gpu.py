@@ -81,11 +81,12 @@ def test_fused_layernorm_modulation_quant_bit_exact(gpu, affine):
 
 
 @pytest.mark.parametrize("Mp,M,N,K,stream_k", [(1408, 1392, 3072, 3072, True), (384, 300, 384, 256, False),
-                                               (512, 464, 512, 14336, True)])
+                                               (2688, 2640, 3072, 256, False), (512, 464, 512, 14336, True)])
 def test_layernorm_partials_of_the_residual_epilogue(gpu, Mp, M, N, K, stream_k):
     """The gated-residual epilogue's LayerNorm chunk partials of the rows it writes, bit-exact to the oracle's
     partials of those rows, through each launch that runs the residual: the balanced form with its 32 x 32 pieces
-    (1392 x 3072, K 3072), the one-pass tile, stream-K + merge (K 14336). Then the LayerNorm-fused quantizer of the
+    (1392 x 3072, K 3072), the pieces of few tokens (300 x 384), the one-pass tile (2640 x 3072: more pieces than 6 a
+    CU), stream-K + merge (K 14336). Then the LayerNorm-fused quantizer of the
     new rows from those partials equals the quantizer forming them itself (and the oracle), bit for bit."""
     from wdl import ops, w4a4
 
@@ -189,9 +190,10 @@ def test_scale_pairs_are_exact_for_every_fp16_and_bf16_scale(gpu):
 
 @pytest.mark.parametrize("sdt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,N,K,valid", [(128, 256, 512, 100), (256, 128, 3072, 256), (1408, 384, 3072, 1392),
-                                         (2688, 384, 3072, 2640)])
+                                         (2688, 384, 3072, 2640), (2688, 3072, 576, 2640), (1024, 3072, 256, 1000)])
 def test_gemm_scaled_lowrank_bias_matches_oracle(gpu, M, N, K, valid, sdt):
-    """bf16 and fp16 weight scales (the two modes; fp16 goes through the exact hi + lo pair)."""
+    """bf16 and fp16 weight scales (the two modes; fp16 goes through the exact hi + lo pair): the pieces of few tokens
+    (996 at most, the first four shapes) and the tiles (7968 and 3072 pieces, more than 6 a CU)."""
     from wdl import w4a4
 
     g = torch.Generator().manual_seed(7 + M)
@@ -293,10 +295,11 @@ def test_gemm_of_few_tokens_equals_the_same_rows_of_a_large_one(gpu, M, N, K):
             assert torch.equal(parts[0], parts[1][:M]), (M, N, K)
 
 
-def test_gemm_residual_and_gelu_epilogues(gpu):
+@pytest.mark.parametrize("M,N,K", [(256, 256, 512), (2048, 2304, 512)])
+def test_gemm_residual_and_gelu_epilogues(gpu, M, N, K):
+    """In the pieces of few tokens and in the tiles (288 of them, 4608 pieces)."""
     from wdl import w4a4
 
-    M, N, K = 256, 256, 512
     g = torch.Generator().manual_seed(9)
     qa = torch.randint(-7, 8, (M, K), generator=g, dtype=torch.int32)
     qw = torch.randint(-8, 8, (N, K), generator=g, dtype=torch.int32)

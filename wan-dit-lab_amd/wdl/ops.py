@@ -222,7 +222,7 @@ def gemm_launch(q, ascales, lora, wcodes, wscales, proj_up, bias, M, out, epilog
                 stream_k=True, ln_out=None):
     """W4A4 GEMM on the quantizer's outputs (q, ascales, lora) and tile-blocked fp6 weight codes (weight_codes);
     wscales: the scale pairs (scale_pairs), or bf16 / fp16 scales (converted once per tensor, cached_scale_pairs).
-    stream_k=False runs the one-pass launch also for the shapes that the library splits in K. ln_out (with the
+    stream_k=False leaves no shape split in K: the one-pass launch's sums, for few tokens in 32 x 32 pieces. ln_out (with the
     gated residual): fp32 [M, N / 32, 2] receiving the LayerNorm chunk partials of the updated rows of out."""
     wscales = cached_scale_pairs(wscales)
     if q.dim() != 4 or wcodes.dim() != 4 or q.shape[2:] != (BLOCK, ROW6) or wcodes.shape[2:] != (BLOCK, ROW6):
