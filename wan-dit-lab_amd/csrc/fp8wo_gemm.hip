@@ -16,12 +16,15 @@
 // with an explicit vmcnt):
 //   W stage: [features][64 B] of e4m3, each row's four 16-byte quarters XOR-swizzled by (row / 4) % 4;
 //   X stage: [128 tokens][128 B] of bf16, each row's eight 16-byte chunks XOR-swizzled by (row / 2) % 8,
-// so the 8- and 16-byte fragment reads of 16 consecutive rows cover the banks once. Fragments are double-buffered in
+// which spreads the 8- and 16-byte fragment reads of 16 consecutive rows over the banks. Fragments are double-buffered in
 // registers across steps and stages. Rows of X past M are loaded from row M - 1 (never written back).
 //
-// What bounds it: the operands' way into LDS (a timing copy without the loads: 2640 x 9216 x 3072 in 115 us; the matrix
-// cores alone allow 70). Measured (graph replays, one box): 2640 tokens QKV 184 -> 147 us (1.02 PFLOP/s; 8192^3 in
-// bf16 through the library GEMM 1.25), o 62.8 -> 50.7; 1392 tokens QKV 108 -> 89, o 48.7 -> 39.5 us. The steps: fragments
+// What bounds it: no single unit. The matrix cores are busy for half of the time at 2640 x 9216 x 3072 (they alone would
+// take 70 us); a third of the wave cycles wait at the ring's barrier and loads, a third for their turn to issue, LDS waits
+// are 1 % (bank conflicts one cycle per active one). A timing copy without the loads takes 115 us, so the operands' way
+// into LDS is the largest part that can be named. Measured (graph replays, both sides in turn on one box): 2640 tokens QKV
+// 177 -> 141 us (1.06 PFLOP/s; 8192^3 in bf16 through the library GEMM 1.25), o 61.2 -> 48.5; 1392 tokens QKV 104 -> 85, o
+// 47.7 -> 37.7; 464 tokens QKV 48.4 -> 37.6, o 35.1 -> 27.0 us. The steps, as each was made: fragments
 // double-buffered and the one-instruction widening -8 % at 1392 tokens; the 256 x 128 tiles -12 % at 2640; rows staged to
 // whole segments on the way out and the swizzle by row / 2 the rest.
 #include "wdl_common.h"

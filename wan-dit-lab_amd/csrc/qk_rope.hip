@@ -71,9 +71,10 @@ __device__ __forceinline__ void load8(const uint16_t* p, float* f) {
 //
 // Bound: Q and K are read and written once, 34 MB at 1392 tokens x 24 heads (7.1 us at the card's copy rate). The
 // rows are short, so what a wave does beside moving them decides: with the table entries loaded and held for each
-// chunk (48 extra registers in fp64) and the grid place from 64-bit divisions it was 12.8 us there (19.6 at 2640
-// tokens, 6.7 at 464); with one set of entries per lane and 32-bit divisions 10.2
-// (15.7 and 5.6).
+// chunk (48 extra registers in fp64) and the grid place from 64-bit divisions it was 12.8 us there (18.9 at 2640
+// tokens, 7.0 at 464; with an fp64 table 15.8, 23.8 and 8.2); with one set of entries per lane and 32-bit divisions
+// 10.2 (15.4 and 5.9; fp64 11.8, 17.5 and 6.6). Counters at 1392 tokens: 645 vector instructions a wave (fp64 693), 45 %
+// of the wave cycles wait for loads and 26 % for their turn to issue.
 template <typename T>
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(NormRopeArgs a) {
     constexpr int CW = MAXCH / 2;  // chunks per lane and wave

@@ -577,9 +577,12 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a) {
 
 // Few tiles (at most half the CUs) over long keys: each tile's key blocks in this many equal shares of 8 blocks or more, one
 // workgroup each, where that takes 32 blocks or more off a workgroup's chain (0.57 us each; the partial states and the
-// merge launch cost up to 18 us), 1 for none. Measured (us, whole tiles -> split): 464 queries x 24 heads (96 tiles, 2
-// shares) over 9744 keys 100.1 -> 73.9, over 2784 keys (44 blocks) 38.4 -> 42.5, hence the line; 12 heads (5 shares) over
-// 9744 keys 99.3 -> 44.5; 128 x 24 heads (10) 99.3 -> 34.4; 64 x 12 heads over 4096 keys (8) 46.7 -> 24.3.
+// merge launch cost up to 18 us), 1 for none. Measured (us, graph replays, whole tiles -> split): 464 queries x 24 heads
+// (96 tiles, 2 shares) over 9744 keys 100.3 -> 71.7; 12 heads (5 shares) 99.6 -> 41.5; 128 x 24 heads (10) 99.4 -> 33.2; 64
+// x 12 heads over 4096 keys (8) 46.8 -> 23.9. Near the line, where the gain is least: 96 tiles over 63 / 67 / 79 blocks 48.9
+// -> 46.0, 51.0 -> 46.7, 57.9 -> 50.0; 128 tiles (2) over 63 blocks 49.3 -> 48.3; 72 tiles (3) over 47 blocks 39.1 -> 38.2;
+// 64 tiles (4) over 42 blocks 36.0 -> 33.5; 48 tiles (5) over 40 blocks 34.8 -> 30.7; and below it 96 tiles over 44 blocks
+// (2) 38.4 -> 42.5.
 int64_t few_shares(int64_t T, int64_t nblk) {
     const int64_t cus = cu_count();
     if (cus <= 0 || cus > MAX_WG || 2 * T > cus) return 1;

@@ -1139,7 +1139,7 @@ __device__ __forceinline__ auto buffer_of(const void* base, int64_t bytes) {
 // is one scalar offset: no vector address arithmetic), two batches of FEW_GROUPS groups in turn, and the products of a
 // group run on the matrix core while the previous group's are added. Left to itself the compiler put each product
 // before its own adds and waited for it, with some 40 address instructions a group: 12.5 us for one token at N = K = 3072
-// against 7.2 now; batches of 3 take the same time, of 6 and 8 (twice the registers, one wave a SIMD) up to 1.5 times
+// against 7.5 now (of the wave cycles there 57 % issue and 32 % wait); batches of 3 take the same time, of 6 and 8 (twice the registers, one wave a SIMD) up to 1.5 times
 // as long where there are more than 4 pieces a CU.
 constexpr int FEW_GROUPS = 4;
 template <int EPI>
@@ -1360,9 +1360,9 @@ int64_t sk_shares(int64_t Mp, int64_t N, int64_t K) {
 }
 
 // Few pieces: with 128 x 128 tiles a few tokens give 24 workgroups at N = 3072, each going through K on one CU. Measured
-// (us; tiles -> pieces): N = K = 3072: 1 token 16.7 -> 7.2, 77 17.1 -> 9.3, 464 (5.6 pieces a CU) 17.6 -> 16.0; N =
-// 9216: 128 tokens (4.5) 17.5 -> 13.4, 200 (7.9) 18.1 -> 20.8; N = 16384, K = 512: 33 (4) 6.6 -> 5.5, 77 (6) 6.9 -> 6.9,
-// 128 (8) 7.1 -> 8.7; N = K = 1536: 464 tokens (2.8) 11.0 -> 7.3. Pieces read each operand row once per 32 of the
+// (us; tiles -> pieces): N = K = 3072: 1 token 17.0 -> 7.5, 77 17.4 -> 9.5, 464 (5.6 pieces a CU) 18.0 -> 16.8, 512 (6)
+// 17.8 -> 16.4; N = 9216: 128 tokens (4.5) 17.5 -> 13.4, 200 (7.9) 18.1 -> 20.8; N = 16384, K = 512: 33 (4) 6.6 -> 5.5,
+// 77 (6) 6.9 -> 6.9, 128 (8) 7.1 -> 8.7; N = K = 1536: 464 tokens (2.8) 11.0 -> 7.3. Pieces read each operand row once per 32 of the
 // other side, so the tiles win from 6 pieces a CU on. Where stream-K would run, a piece's whole K is the chain: N =
 // 1536, K = 7168: 77 tokens 38.7 -> 13.6, 464 (2.8) 25.3 -> 18.3; N = 3072, K = 8192: 300 (3.8) 28.2 -> 23.4, 464
 // (5.6) 31.7 -> 37.6; K = 14336: 77 29.2 -> 32.4; N = 1024, K = 28672: 42.2 -> 46.1; hence up to K = 128 groups and 3
