@@ -1,12 +1,13 @@
-"""Kernel timings at the step's shapes, for profiling runs: `python kbench.py attention|cross|prep|gemm|quant
-[lib]`.
+"""Kernel timings at the step's shapes, for profiling runs: `python kbench.py
+attention|chunk|cross|prep|gemm|few|quant|rope|fp8|fp8wo [lib]`.
 
 attention: Sage prep + attention of 1280 and 1392 queries over a full 9744-key window (8352 cached FP8 tokens + the
 chunk), 24 x 128 heads; prep: the Sage preparation (K mean and V maxima, int8 K and fp8 V of the whole window) of
 the same two shapes; gemm: the W4A4 GEMMs of one block at 1392 tokens (QKV 3072 -> 9216, o 3072 -> 3072 with the
 gated residual, FFN-up 3072 -> 14336 with GELU (bf16 out) and fused with the second layer's quantization, FFN-down 14336 -> 3072 with the gated residual), random weights; quant: the activation quantizer with its low-rank down projection at 1392 tokens
 (K 3072 with the fused LayerNorm and modulation, its statistics formed in the launch or from chunk partials given,
-K 3072 plain, K 14336 unsigned).
+K 3072 plain, K 14336 unsigned); few: W4A4 products of few tokens, and the attention of few query tiles split over the
+keys and in whole tiles; rope: the Q / K norm and rotation at 464, 1392 and 2640 tokens.
 Each shape is captured into a HIP graph of 10 launches and replayed; one line per shape with microseconds per
 launch (gemm: the launch the library picks and the one-pass launch, alternated three times, the best of each).
 An optional library path replaces lib/libwdl.so (for comparing builds).
@@ -227,15 +228,61 @@ def quant():
         print(f"quant {name} {M}x{K}: {us:.1f} us ({M * K * 2 / us / 1e3:.0f} GB/s of x)", flush=True)
 
 
+def few():
+    import torch
+
+    from wdl import _lib, ops, w4a4
+
+    dev = "cuda"
+    g = torch.Generator(device=dev).manual_seed(0)
+    for M, N, K in ((1, 3072, 3072), (77, 3072, 3072), (464, 3072, 3072), (512, 3072, 3072), (77, 1536, 7168)):
+        t = w4a4.random_parts(N, K, dev, g)
+        wc, wsp = ops.as_codes(t["qweight"], K), ops.scale_pairs(t["wscales"])
+        x = torch.randn(M, K, device=dev, generator=g).to(torch.bfloat16)
+        q, asc, lora = ops.act_quant_launch(x, t["smooth"], t["proj_down"])
+        out = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
+        us = _replay_us(lambda: ops.gemm_launch(q, asc, lora, wc, wsp, t["proj_up"], t["bias"], M, out))
+        print(f"few tokens {M}x{N}x{K}: {us:.1f} us", flush=True)
+    for n, H, L in ((464, 24, 4096), (464, 24, 9744), (464, 12, 9744), (128, 24, 9744), (64, 12, 4096)):
+        K, V = (torch.randn(L, H * 128, device=dev, generator=g).to(torch.bfloat16) for _ in range(2))
+        Q = torch.randn(n, H * 128, device=dev, generator=g).to(torch.bfloat16)
+        none, one = torch.zeros(1, 1, H, 128, device=dev, dtype=torch.uint8), torch.ones(1, 1, H, 1, device=dev)
+        p = ops.sage_prep_launch(none, one, none, one, K, V, 0)
+        out = torch.empty_like(Q)
+        split = _replay_us(lambda: ops.sage_attn_q16_launch(Q, p, L, 128 ** -0.5, out))
+        whole = _replay_us(lambda: _lib.host().sage_attn_q16(Q, p["k"], p["k_scale"], p["v"], p["v_scale"], L,
+                                                             128 ** -0.5, out, 0, None, ops.stream_of(Q)))
+        print(f"few tiles n={n} heads={H} L={L}: {split:.1f} us in {_lib.library().wdl_sage_attn_split(n, L, H)} "
+              f"shares, {whole:.1f} us whole", flush=True)
+
+
+def rope():
+    import torch
+
+    from wdl import ops
+    from wdl.rope import freqs
+
+    dev, H = "cuda", 24
+    g = torch.Generator(device=dev).manual_seed(0)
+    for name, dtype in (("fp64", torch.float64), ("fp32", torch.float32)):
+        table = freqs(device=dev).to(dtype)
+        for M, grid in ((464, (1, 16, 29)), (1392, (3, 16, 29)), (2640, (3, 22, 40))):
+            q, k = (torch.randn(M, H * 128, device=dev, generator=g).to(torch.bfloat16) for _ in range(2))
+            w = torch.rand(H * 128, device=dev, generator=g).to(torch.bfloat16)
+            us = _replay_us(lambda: ops.qk_norm_rope_launch(q, k, w, w, table, grid, 5))
+            print(f"norm + rope of Q and K {M}x{H * 128}, {name} table: {us:.1f} us "
+                  f"({8 * M * H * 128 / us / 1e3:.0f} GB/s)", flush=True)
+
+
 def main(argv):
-    if len(argv) < 2 or argv[1] not in ("attention", "chunk", "cross", "prep", "gemm", "quant", "fp8", "fp8wo"):
-        raise SystemExit("usage: python kbench.py attention|chunk|cross|prep|gemm|quant|fp8|fp8wo [library path]")
+    modes = {f.__name__: f for f in (attention, chunk, cross, prep, gemm, few, quant, rope, fp8, fp8wo)}
+    if len(argv) < 2 or argv[1] not in modes:
+        raise SystemExit(f"usage: python kbench.py {'|'.join(modes)} [library path]")
     if len(argv) > 2:
         from wdl import _lib
 
         _lib.LIB_PATH = Path(argv[2])
-    {"attention": attention, "chunk": chunk, "cross": cross, "prep": prep, "gemm": gemm, "quant": quant, "fp8": fp8,
-     "fp8wo": fp8wo}[argv[1]]()
+    modes[argv[1]]()
 
 
 if __name__ == "__main__":

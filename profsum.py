@@ -20,8 +20,10 @@ import re
 import sys
 
 KERNELS = re.compile(r"(w4a4_gemm_kernel<[^>]*>|w4a4_gemm_sk_kernel<[^>]*>|w4a4_gemm_bal_kernel<[^>]*>|"
-                     r"w4a4_merge_kernel<[^>]*>|attn_merge_kernel|"
-                     r"sage_attn_kernel|quant_kernel|quant_kv_kernel|colstats_kernel|"
+                     r"w4a4_merge_kernel<[^>]*>|w4a4_few_kernel<[^>]*>|fp8wo_gemm_kernel<[^>]*>|"
+                     r"fp8_gemm_kernel<[^>]*>|fp8_gemm_sk_kernel<[^>]*>|attn_bf16_kernel<[^>]*>|attn_bf16_prep_kernel|"
+                     r"attn_merge_kernel|rows_kernel<[^>]*>|tensor_max_kernel<[^>]*>|tensor_quant_kernel<[^>]*>|"
+                     r"sage_attn_kernel|quant_kernel|quant_kv_kernel|colstats_kernel|lora_sum4_kernel|"
                      r"qk_norm_rope_kernel|quant_q_kernel|row_stats_kernel|lora_sum_kernel|kv_append_kernel<[^>]*>|"
                      r"finalize_kernel|bitwise_not)")
 
