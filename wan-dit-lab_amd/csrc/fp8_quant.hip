@@ -14,6 +14,8 @@
 //         has to start zeroed.
 #include "wdl_common.h"
 
+#include <type_traits>
+
 namespace {
 
 using namespace wdl;
@@ -54,8 +56,16 @@ __device__ __forceinline__ void ld8<uint16_t>(const uint16_t* p, float* f) {
 
 // x / s for the quantizers' scale s (its reciprocal rs beside it): div_rn, the IEEE quotient wherever it does not round
 // to a zero code; an infinite s (an infinite |x|) takes the division itself (finite values: 0, infinite: NaN)
+template <bool FINITE>
 __device__ __forceinline__ float quotient(float x, float s, float rs) {
-    return s < INFINITY ? div_rn(x, s, rs) : x / s;
+    return FINITE ? div_rn(x, s, rs) : x / s;
+}
+// codes(true_type) for a finite scale (one value in a wave: a scalar branch), codes(false_type) for an infinite one. A
+// choice per value put two branches between the quotients: rows of 1536 values took 3.8 us for 3.6.
+template <typename Codes>
+__device__ __forceinline__ void by_scale(float s, Codes codes) {
+    if (__uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(s))) < INFINITY) codes(std::true_type{});
+    else codes(std::false_type{});
 }
 
 // One workgroup of WPR waves per row, 8 values per lane and step, two steps in flight: the row's maximum (lanes,
@@ -102,19 +112,21 @@ __global__ __launch_bounds__(64 * WPR) void rows_kernel(const T* x, int64_t ldx,
     const float s = fmaxf(amax, 1e-12f) / FP8_MAX;
     if (t == 0) scale[row] = s;
     const float rs = 1.0f / s;
-    auto codes = [&](int64_t cc) {
-        float f[8];
-        ld8<T>(xr + 8 * cc, f);
+    by_scale(s, [&](auto finite) {
+        auto codes = [&](int64_t cc) {
+            float f[8];
+            ld8<T>(xr + 8 * cc, f);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) f[e] = quotient(f[e], s, rs);
-        qr[cc] = make_uint2(e4m3x4(f), e4m3x4(f + 4));
-    };
-    c = t;
-    for (; c + NT < chunks; c += 2 * NT) {
-        codes(c);
-        codes(c + NT);
-    }
-    if (c < chunks) codes(c);
+            for (int e = 0; e < 8; ++e) f[e] = quotient<decltype(finite)::value>(f[e], s, rs);
+            qr[cc] = make_uint2(e4m3x4(f), e4m3x4(f + 4));
+        };
+        int64_t c = t;
+        for (; c + NT < chunks; c += 2 * NT) {
+            codes(c);
+            codes(c + NT);
+        }
+        if (c < chunks) codes(c);
+    });
 }
 
 // Chunk i (8 values) of a [rows, K] matrix with row stride ldx. FLAT: ldx = K, so the chunks are consecutive (a 64-bit
@@ -162,23 +174,25 @@ __global__ __launch_bounds__(256) void tensor_quant_kernel(const T* x, int64_t l
     const float rs = 1.0f / s;
     const int64_t k8 = K / 8, n8 = M * k8, np8 = Mp * k8, stride = int64_t(gridDim.x) * 256;
     uint2* const out = reinterpret_cast<uint2*>(q);  // [Mp, K] bytes, no gaps: chunk i is out[i]
-    int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    for (; i < n8; i += INFLIGHT * stride) {
-        float f[INFLIGHT][8];
+    const int64_t first = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    by_scale(s, [&](auto finite) {
+        for (int64_t i = first; i < n8; i += INFLIGHT * stride) {
+            float f[INFLIGHT][8];
 #pragma unroll
-        for (int u = 0; u < INFLIGHT; ++u)
-            ld8<T>(chunk_at<FLAT>(x, ldx, k8, i + u * stride < n8 ? i + u * stride : i), f[u]);
+            for (int u = 0; u < INFLIGHT; ++u)
+                ld8<T>(chunk_at<FLAT>(x, ldx, k8, i + u * stride < n8 ? i + u * stride : i), f[u]);
 #pragma unroll
-        for (int u = 0; u < INFLIGHT; ++u) {
+            for (int u = 0; u < INFLIGHT; ++u) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                f[u][e] = quotient(f[u][e], s, rs);
-                if constexpr (sizeof(T) == 2) f[u][e] = bf16_to_f32(f32_to_bf16(f[u][e]));
+                for (int e = 0; e < 8; ++e) {
+                    f[u][e] = quotient<decltype(finite)::value>(f[u][e], s, rs);
+                    if constexpr (sizeof(T) == 2) f[u][e] = bf16_to_f32(f32_to_bf16(f[u][e]));
+                }
+                if (i + u * stride < n8) out[i + u * stride] = make_uint2(e4m3x4(f[u]), e4m3x4(f[u] + 4));
             }
-            if (i + u * stride < n8) out[i + u * stride] = make_uint2(e4m3x4(f[u]), e4m3x4(f[u] + 4));
         }
-    }
-    for (i = n8 + int64_t(blockIdx.x) * 256 + threadIdx.x; i < np8; i += stride) out[i] = make_uint2(0u, 0u);
+    });
+    for (int64_t i = n8 + int64_t(blockIdx.x) * 256 + threadIdx.x; i < np8; i += stride) out[i] = make_uint2(0u, 0u);
 }
 
 int tensor_blocks(int64_t M, int64_t K) {
