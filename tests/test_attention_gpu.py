@@ -121,6 +121,27 @@ def test_prep_with_append_is_store_then_prep(gpu, at, n, H):
         assert torch.equal(pa[key], pb[key]), key
 
 
+@pytest.mark.parametrize("cached", [False, True])
+@pytest.mark.parametrize("splits", [1, 2, 15, 17, 32, 33])
+def test_prep_of_exact_sums_is_the_same_for_any_number_of_splits(gpu, splits, cached):
+    """A call's partial sums are added a batch of 16 at a time, a batch cut short included: over multiples of 1/8, whose
+    sums are exact in fp32, every number of splits gives the same bits."""
+    from wdl import _lib, ops, sage_kv
+
+    g = torch.Generator().manual_seed(splits)
+    at, n, H = 100, 333, 3
+    k, v = (torch.randint(-8, 9, (1, at, H, 128), generator=g).div(8).to(torch.float8_e4m3fn).cuda() for _ in range(2))
+    one = torch.ones(1, at, H, 1, device="cuda")
+    K, V = (torch.randint(-24, 25, (n, H * 128), generator=g).div(8).to(torch.bfloat16).cuda() for _ in range(2))
+    stats = sage_kv.cache_stats(k, one, v, one, at) if cached else None
+    run = lambda s: _lib.host().sage_prep(k.view(torch.uint8), one, v.view(torch.uint8), one, K, V, at, s, stats, False,
+                                          ops.stream_of(K))
+    assert all(torch.equal(a, b) for a, b in zip(run(splits), run(16)))
+    mean = run(splits)[4].double().cpu()
+    want = (k[0].double().sum(0) + K.view(n, H, 128).double().sum(0)).cpu() / (at + n)
+    assert torch.equal(mean, want.float().double())
+
+
 def test_attend_with_append_refuses_before_writing(gpu):
     """sage_kv.attend(append=True) checks the store's requirements (rows past the cache here) before any launch."""
     from wdl import sage_kv

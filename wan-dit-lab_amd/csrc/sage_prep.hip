@@ -134,15 +134,25 @@ __global__ __launch_bounds__(256) void colstats_kernel(Src k, Src v, int64_t H, 
     }
 }
 
-// The splits' partial sums (or maxima) of one column added in increasing order onto `from`; the loads of a batch of 16
-// are all issued before the first is used (one memory round trip per batch, not one per split).
+// The splits' partial sums (or maxima) of column i added in increasing order onto `from`; the loads of a batch of 16
+// are all issued before the first is used (one memory round trip per batch, not one per split). The splits' rows are
+// scalar addresses and i a 32-bit offset in them, so a whole batch takes a load and an add per split and no address
+// arithmetic on the vector unit, which quant_kv_kernel needs for its values.
 template <typename Op>
-__device__ __forceinline__ float over_splits(const float* part, int S, int64_t stride, float from, Op op) {
+__device__ __forceinline__ float over_splits(const float* part, uint32_t i, int S, int64_t stride, float from, Op op) {
     constexpr int BATCH = 16;
-    for (int s0 = 0; s0 < S; s0 += BATCH) {
+    int s0 = 0;
+    for (; s0 + BATCH <= S; s0 += BATCH) {
         float p[BATCH];
 #pragma unroll
-        for (int j = 0; j < BATCH; ++j) p[j] = s0 + j < S ? part[(s0 + j) * stride] : 0.0f;
+        for (int j = 0; j < BATCH; ++j) p[j] = (part + (s0 + j) * stride)[i];
+#pragma unroll
+        for (int j = 0; j < BATCH; ++j) from = op(from, p[j]);
+    }
+    if (s0 < S) {
+        float p[BATCH];
+#pragma unroll
+        for (int j = 0; j < BATCH; ++j) p[j] = (part + (s0 + j < S ? s0 + j : s0) * stride)[i];
 #pragma unroll
         for (int j = 0; j < BATCH; ++j)
             if (s0 + j < S) from = op(from, p[j]);
@@ -164,19 +174,19 @@ struct Stats {
     const float* base;
     int S;
     // K sum / |V| maximum of column i = h D + d
-    __device__ __forceinline__ float sum(int64_t i, int64_t HD) const {
-        return over_splits(part_k + i, S, HD, base ? base[i] : 0.0f, Add{});
+    __device__ __forceinline__ float sum(uint32_t i, int64_t HD) const {
+        return over_splits(part_k, i, S, HD, base ? base[i] : 0.0f, Add{});
     }
-    __device__ __forceinline__ float max(int64_t i, int64_t HD) const {
-        return over_splits(part_v + i, S, HD, base ? base[HD + i] : 0.0f, Max{});
+    __device__ __forceinline__ float max(uint32_t i, int64_t HD) const {
+        return over_splits(part_v, i, S, HD, base ? (base + HD)[i] : 0.0f, Max{});
     }
 };
 
 // wdl_sage_cache_stats: the sums and maxima themselves, [2][H][D]
 __global__ void finalize_kernel(Stats st, int64_t HD, float* out) {
-    const int64_t i = int64_t(blockIdx.x) * D + threadIdx.x;
+    const uint32_t i = blockIdx.x * D + threadIdx.x;
     out[i] = st.sum(i, HD);
-    out[HD + i] = st.max(i, HD);
+    (out + HD)[i] = st.max(i, HD);
 }
 
 __device__ __forceinline__ int v_position(int t) { return 32 * ((t % 8) / 4) + 4 * (t / 8) + t % 4; }
@@ -262,7 +272,7 @@ __global__ __launch_bounds__(256) void quant_kv_kernel(Src k, Src v, int64_t H, 
     // the head's statistics from the splits' partials (16 KB from L2 per workgroup, beside its tokens' loads; a launch
     // of its own for them took 4 - 5 us in front of this one); the first block keeps them for the caller
     {
-        const int64_t i = h * D + t % D;
+        const uint32_t i = blockIdx.y * D + t % D;
         if (t < D) {
             const float mean = st.sum(i, H * D) / float(L);
             stat[0][t] = mean;
