@@ -270,7 +270,9 @@ __global__ __launch_bounds__(256) void quant_kv_kernel(Src k, Src v, int64_t H, 
     const int t = threadIdx.x, tt = t / 4, dq = (t % 4) * 32;
     const int64_t tok = blk * 64 + tt;
     // the head's statistics from the splits' partials (16 KB from L2 per workgroup, beside its tokens' loads; a launch
-    // of its own for them took 4 - 5 us in front of this one); the first block keeps them for the caller
+    // of its own for them took 4 - 5 us in front of this one: 464 tokens beside 928 cached ones, 24 heads, from cached
+    // statistics 13.8 -> 11.8 us, 1392 beside 8352 32.8 -> 30.9, 2640 beside 15840 51.9 -> 53.2); the first block keeps
+    // them for the caller
     {
         const uint32_t i = blockIdx.y * D + t % D;
         if (t < D) {
